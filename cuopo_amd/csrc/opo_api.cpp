@@ -112,6 +112,8 @@ struct Group {
   int phase_mode = -1;                    // linear phase: -1 auto, 0 full table, 1 factorised
   double tuned_us = 0;                    // slice time of the autotuner's choice (0 = not tuned)
   bool any_gdd = false;
+  opo::ResSync *d_sync = nullptr;  // counters of the resident pass; null: no resident pass for this group
+  int *d_err = nullptr;            // its time-out flag
   std::vector<void *> allocs;
   // no-allocation mode: device memory comes from the caller's buffers (fields,
   // pump) and a bump pool over the static scratch array instead of hipMalloc
@@ -133,6 +135,8 @@ struct Engine {
   bool compact = true;  // shrink the launches to the still-active instances during a converging run
   int accel_every = 0;     // round-trip extrapolation every this many round trips (0: off), see accel_step
   int accel_start = 1000;  // ... from this many round trips of the run on
+  bool resident = true;  // crystal passes as one launch where every group allows it (opo_resident.h)
+  bool forked = false;   // the groups' chains run on their own streams (fork_groups .. join_groups)
   bool save_enabled = false;
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -333,6 +337,12 @@ int make_group(Engine &E, Group &g) {
   } else {
     HIPCHK(hipMemsetAsync(g.d_hist, 0, (size_t)n * g.hist_len * sizeof(double), E.stream));
   }
+  if (E.resident && opo::resident_supported(g.N1, g.N2, 8, 8)) {
+    RCHK(dalloc(g, (void **)&g.d_sync, sizeof(opo::ResSync)));
+    RCHK(dalloc(g, (void **)&g.d_err, 8));
+    const int e = opo::launch_zero(g.d_err, 1, E.stream);
+    if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
+  }
   g.inst.resize(n);
   for (int k = 0; k < n; ++k) {
     Instance &I = g.inst[k];
@@ -506,6 +516,7 @@ OpoInst make_desc(const Engine &E, const Group &g, int k) {
   d.power_hist = g.d_hist + (size_t)k * g.hist_len; d.hist_len = g.hist_len;
   d.conv_rt = g.d_conv + k; d.p_ref = g.d_pref + k; d.p_first = g.d_pfirst + k; d.r_prev = g.d_rprev + k; d.status = g.d_status + k;
   d.snap = I.snap;
+  for (int k2 = 0; k2 < 2; ++k2) d.lfac_spt[k2] = I.use_fac && group_factored(g) ? I.lfac[k2] : nullptr;
   d.active_v = 1;
   return d;
 }
@@ -524,6 +535,124 @@ int sync_insts(Engine &E) {
   return OPO_OK;
 }
 
+// ------------------------------------------------------------ resident pass
+
+// Shape of the resident pass over `count` instances of a group: samples per
+// thread of its transforms, teams per XCD, tiles a block holds side by side,
+// blocks per XCD (one per CU: a barrier costs less with fewer, larger blocks).
+struct ResShape {
+  int ce, re, teams, sub, blocks;
+};
+constexpr int kXcdCus = 32, kMaxSub = 4;
+
+// The samples per thread are the group's, as the two-launch path runs them, so
+// both paths give the same bits.
+ResShape res_shape(const Group &g, int count) {
+  ResShape r{g.ce, g.re, 1, 1, kXcdCus};
+  const int need = (count + opo::kXcds - 1) / opo::kXcds;  // instances per XCD
+  const int tiles = g.N / (64 * std::min(r.ce, r.re));     // of the stage with more tiles
+  while (r.teams < need && 2 * r.teams <= opo::kMaxTeams && r.teams * tiles < kMaxSub * kXcdCus) r.teams *= 2;
+  while (r.sub < kMaxSub && r.sub * kXcdCus < r.teams * tiles) r.sub *= 2;
+  r.blocks = std::min(kXcdCus, std::max(r.teams, r.teams * tiles / r.sub));
+  return r;
+}
+
+// The halves of a large one-size batch (split_large_group) share one resident
+// pass, launched with the first.
+const Group *res_second(const Engine &E, const Group &g) {
+  return E.groups.size() == 2 && &g == &E.groups[0] && E.groups[1].N == g.N ? &E.groups[1] : nullptr;
+}
+bool res_follower(const Engine &E, const Group &g) { return E.groups.size() == 2 && &g == &E.groups[1] && E.groups[0].N == g.N; }
+int res_count(const Engine &E, const Group &g) {  // instances the pass runs
+  const Group *h = res_second(E, g);
+  return g.launch_n + (h ? h->launch_n : 0);
+}
+ResShape res_shape(const Engine &E, const Group &g) { return res_shape(g, res_count(E, g)); }
+
+// Whether the crystal passes run resident: one grid size, N = 2^10 .. 2^15,
+// and few enough instances still running.  Measured per slice on an MI355X, resident against
+// the autotuned two-launch path (CW three equations, FP64): 1 instance 5.3
+// against 6.8 us at 2^12, 7.0 against 8.2 at 2^14, 9.9 against 9.8 at 2^15;
+// 8 instances 7.6 against 15.0 at 2^14; 2^19 samples in all 1.3 to 2.1 times
+// faster at every grid.  Beyond
+// that the teams run several turns of 2^19 samples, about 16.5 us each
+// whether full or not, and the two-launch path streams about 31 ps per sample
+// beside 7 us; the shorter estimate decides (256
+// instances of 2^14: 124 against 141 us; 71: 49 against 41).
+// FP32C streams half the bytes on the two-launch path and the pass is bound by
+// arithmetic there, so it ends at 2^19 samples (1.05 to 1.7 times; 0.5 to 1.2
+// beyond); with 4 samples per thread at 2^15 its 128 tiles per stage lose at
+// any count up to 9 (0.75 to 0.84).
+// Several grid sizes run side by side on their streams, where the passes would
+// run one after another (0.8 to 1.0 times).
+constexpr long long kResTurn = 1LL << 19;  // samples of one turn of every XCD's teams
+constexpr double kResTurnUs = 16.5, kStreamUs = 7.0, kStreamUsPerSample = 31e-6;
+
+bool engine_resident(const Engine &E) {
+  if (!E.resident || E.groups.empty()) return false;
+  const Group &g = E.groups[0];
+  if (!g.d_sync || (E.groups.size() != 1 && !res_second(E, g))) return false;
+  for (const auto &h : E.groups)
+    if (!opo::resident_supported(h.N1, h.N2, h.ce, h.re)) return false;
+  const int count = res_count(E, g);
+  const long long samples = (long long)count * g.N;
+  if (g.fp32) return samples <= kResTurn && !(g.N == (1 << 15) && std::min(g.ce, g.re) == 4);
+  if (samples <= kResTurn) return true;
+  const ResShape r = res_shape(g, count);
+  const int turn = r.teams * opo::kXcds;
+  return (count + turn - 1) / turn * kResTurnUs < kStreamUs + kStreamUsPerSample * (double)samples;
+}
+
+// 8-byte words of the counters that a pass of this shape uses
+int res_sync_words(const ResShape &r) {
+  return (int)((offsetof(opo::ResSync, team) + sizeof(opo::ResTeam) * (size_t)(r.teams * opo::kXcds)) / 8);
+}
+
+int clear_sync(Group &g, hipStream_t st) {
+  const int e = opo::launch_zero(g.d_sync, (long long)(sizeof(opo::ResSync) / 8), st);
+  return e == 0 ? OPO_OK : fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
+}
+
+// slices 0 .. nz-1 of every instance: row, column, ..., row (no column stage
+// after the last row).  The counters were cleared by the kernel before.
+// `alone`: of this group only (the autotuner, which saves one group's fields).
+int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
+  const Group *second = alone ? nullptr : res_second(E, g);
+  const int total = g.launch_n + (second ? second->launch_n : 0);
+  if ((!alone && res_follower(E, g)) || total == 0) return OPO_OK;
+  const ResShape r = res_shape(g, total);
+  opo::ResArgs a{};
+  a.tw1 = g.tw1; a.tw2 = g.tw2; a.twlo = g.twlo; a.twhi = g.twhi;
+  a.lobits = g.lobits; a.xl_bits = g.xl_bits[eidx(r.re)];
+  a.NZ = nz; a.count = g.launch_n;
+  if (second) { a.insts2 = second->d_insts; a.count2 = second->launch_n; }
+  a.teams = r.teams; a.sub = r.sub; a.expect = r.blocks;
+  a.spread = total < r.teams * opo::kXcds;
+  // consecutive handles prefer different XCDs
+  a.prefer = (int)((reinterpret_cast<uintptr_t>(g.d_insts) >> 12) % opo::kXcds);
+  a.sync = g.d_sync;
+  a.err = g.d_err;
+  const int e = opo::launch_resident(g.fp32, g.N1, g.N2, g.NF, r.ce, r.re, g.d_insts, a, r.blocks * opo::kXcds, g.cur);
+  if (e != 0) return fail(OPO_ERR_HIP, std::string("resident pass launch: ") + hipGetErrorString((hipError_t)e));
+  return OPO_OK;
+}
+
+// A pass whose blocks waited too long for each other left its fields undefined.
+int check_resident(Engine &E) {
+  for (auto &g : E.groups) {
+    if (!g.d_err) continue;
+    int err = 0;
+    HIPCHK(hipMemcpyAsync(&err, g.d_err, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    HIPCHK(hipStreamSynchronize(E.stream));
+    if (err != 0) {
+      const int e = opo::launch_zero(g.d_err, 1, E.stream);
+      if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
+      return fail(OPO_ERR_HIP, "crystal pass timed out on the device");
+    }
+  }
+  return OPO_OK;
+}
+
 // ------------------------------------------------------------ stage emitters
 
 int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int store, int s_end, int s_start,
@@ -538,6 +667,11 @@ int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int 
   a.xcd_pack = g.xcd_pack >= 0 ? g.xcd_pack : E.xcd_pack;
   a.swz = !a.xcd_pack && g.ct * esize(g) < 128 && (g.N2 / g.ct) % 8 == 0;
   a.spt = g.ce;
+  if (engine_resident(E)) {  // the general kernel clears the next pass's counters (the slice-interior one ignores these)
+    const Group &lead = res_follower(E, g) ? E.groups[0] : g;
+    a.zero = reinterpret_cast<unsigned long long *>(lead.d_sync);
+    a.zero_words = res_sync_words(res_shape(E, lead));
+  }
   if (E.solver) {
     const Instance &I = g.inst[0];
     a.direct = 1;
@@ -590,15 +724,25 @@ int emit_start(Engine &E, Group &g) {
   return emit_col(E, g, opo::OP_PUMP | opo::OP_NL_START, A, 0, A, A, 0, 0, 0, 0);
 }
 
+// the slices of a crystal pass between the forward columns after NL(z_0) and
+// the inverse columns before the last NL
+int emit_slices(Engine &E, Group &g) {
+  using namespace opo;
+  if (engine_resident(E)) return emit_resident(E, g, E.NZ);
+  const int A = all_mask(g);
+  for (int s = 0; s < E.NZ && g.launch_n > 0; ++s) {
+    RCHK(emit_row(E, g, false, A));
+    if (s < E.NZ - 1) RCHK(emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, s, s + 1, 0, 0));
+  }
+  return OPO_OK;
+}
+
 // one round trip after emit_start (or after a previous non-final round trip)
 int emit_rt_body(Engine &E, Group &g, bool last, int check_every, double tol) {
   using namespace opo;
-  if (g.launch_n == 0) return OPO_OK;  // every instance of the group has finished (compaction)
   const int A = all_mask(g), SI = si_mask(g), NZ = E.NZ;
-  for (int s = 0; s < NZ; ++s) {
-    RCHK(emit_row(E, g, false, A));
-    if (s < NZ - 1) RCHK(emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, s, s + 1, 0, 0));
-  }
+  RCHK(emit_slices(E, g));
+  if (g.launch_n == 0) return OPO_OK;  // every instance of the group has finished (compaction)
   const unsigned tail = OP_MIRROR | OP_SAVE | OP_POWER | OP_SNAP;
   const unsigned cont = last ? 0u : (OP_PUMP | OP_NL_START);
   const int fwd = last ? 0 : A;
@@ -637,8 +781,12 @@ int reset_counters(Engine &E, int rt0) {
 // stream (forked from and joined back to the engine stream), so the hardware
 // queues overlap the groups' kernels; one group uses the engine stream.
 int fork_groups(Engine &E) {
-  if (E.groups.size() == 1) {
-    E.groups[0].cur = E.stream;
+  // resident passes run one after another: a pass closes its teams with the
+  // blocks that start within 20 us, so beside another one that fills the CUs
+  // it would run with a few blocks only
+  E.forked = E.groups.size() > 1 && !engine_resident(E);
+  if (!E.forked) {
+    for (auto &g : E.groups) g.cur = E.stream;
     return OPO_OK;
   }
   HIPCHK(hipEventRecord(E.fork_ev, E.stream));
@@ -650,7 +798,7 @@ int fork_groups(Engine &E) {
 }
 
 int join_groups(Engine &E) {
-  if (E.groups.size() == 1) return OPO_OK;
+  if (!E.forked) return OPO_OK;
   for (auto &g : E.groups) {
     HIPCHK(hipEventRecord(g.done_ev, g.gs));
     HIPCHK(hipStreamWaitEvent(E.stream, g.done_ev, 0));
@@ -733,6 +881,8 @@ int check_active(Engine &E, bool *alive, bool *changed) {
       g.rt = one_wave_rt;
     }
   }
+  // the first resident pass of a batch that has become small enough for it
+  if (*changed && engine_resident(E)) RCHK(clear_sync(E.groups[0], E.stream));
   return OPO_OK;
 }
 
@@ -935,7 +1085,7 @@ int engine_run(Engine &E, int rt0, int n_rt, int check_every, double tol) {
   }
   // surface a launch-time fault immediately
   HIPCHK(hipGetLastError());
-  return OPO_OK;
+  return check_resident(E);
 }
 
 // A batch of one grid size with at least kSplitMin instances runs as two
@@ -979,6 +1129,8 @@ int engine_init(Engine &E, const opo_params *params, int count) {
   // OPO_SPLIT=0 keeps a large one-grid batch in one group (see split_large_group)
   bool split = true;
   if (const char *sp = std::getenv("OPO_SPLIT")) split = sp[0] != '0';
+  // OPO_RESIDENT=0 launches every stage of a crystal pass by itself
+  if (const char *rs = std::getenv("OPO_RESIDENT")) E.resident = rs[0] != '0';
   E.count = count; E.NZ = p0.NZ; E.three_eqs = p0.three_eqs ? 1 : 0; E.regime = p0.regime;
   E.fp32 = p0.precision == OPO_FP32C; E.device = p0.device;
   E.NRT = 1;
@@ -1167,13 +1319,10 @@ int opo_crystal_pass(opo_solver *s) {
   RCHK(reset_counters(E, 0));
   const int A = all_mask(g);
   RCHK(emit_col(E, g, OP_NL_START, A, 0, A, A, 0, 0, 0, 0));
-  for (int sl = 0; sl < E.NZ; ++sl) {
-    RCHK(emit_row(E, g, false, A));
-    if (sl < E.NZ - 1) RCHK(emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, sl, sl + 1, 0, 0));
-  }
+  RCHK(emit_slices(E, g));
   RCHK(emit_col(E, g, OP_NL_END, A, A, 0, A, E.NZ - 1, 0, 0, 0));
   HIPCHK(hipStreamSynchronize(E.stream));
-  return OPO_OK;
+  return check_resident(E);
 }
 
 int opo_linear_step(opo_solver *s) {
@@ -1357,27 +1506,47 @@ int engine_time_stages(Engine &E, Group &g, int iters, double *col_us, double *r
   return OPO_OK;
 }
 
+// FP32C is tuned on the two-launch path even where the pass runs resident: the
+// samples per thread and the phase source also decide how its results round,
+// and both paths then round alike.
+bool time_resident(const Engine &E) { return engine_resident(E) && !E.fp32; }
+
+// n slices as a round trip of the group runs them, for timing: back-to-back
+// (column, row) pairs, or resident passes of up to NZ slices.
+int time_some_slices(Engine &E, Group &g, int n) {
+  using namespace opo;
+  if (time_resident(E)) {
+    for (int left = n; left > 0;) {
+      const int nz = std::min(left, E.NZ);
+      RCHK(clear_sync(g, g.cur));
+      RCHK(emit_resident(E, g, nz, true));
+      left -= nz;
+    }
+    return OPO_OK;
+  }
+  const int A = all_mask(g);
+  for (int it = 0; it < n; ++it) {
+    RCHK(emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, 0, 1 % E.NZ, 0, 0));
+    RCHK(emit_row(E, g, false, A));
+  }
+  return OPO_OK;
+}
+
 // Average device time of one crystal slice as a round trip runs it: after a
 // warm-up slice, iters back-to-back (column stage, row stage) pairs between
 // two events on the group's stream.  The autotuner's objective.
 int engine_time_slices(Engine &E, Group &g, int iters, double *slice_us) {
-  using namespace opo;
   for (auto &I : g.inst)
     if (!I.uploaded) return fail(OPO_ERR_STATE, "time_slices before upload");
   RCHK(sync_insts(E));
   RCHK(reset_counters(E, 0));
-  const int A = all_mask(g);
   hipEvent_t ev[2] = {nullptr, nullptr};
   int rc = OPO_OK;
   for (auto &e : ev)
     if (rc == OPO_OK && hipEventCreate(&e) != hipSuccess) rc = fail(OPO_ERR_HIP, "event create");
-  auto slice = [&] {
-    const int r = emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, 0, 1 % E.NZ, 0, 0);
-    return r != OPO_OK ? r : emit_row(E, g, false, A);
-  };
-  if (rc == OPO_OK) rc = slice();
+  if (rc == OPO_OK) rc = time_some_slices(E, g, 1);
   if (rc == OPO_OK && hipEventRecord(ev[0], g.cur) != hipSuccess) rc = fail(OPO_ERR_HIP, "event record");
-  for (int it = 0; it < iters && rc == OPO_OK; ++it) rc = slice();
+  if (rc == OPO_OK) rc = time_some_slices(E, g, iters);
   if (rc == OPO_OK && hipEventRecord(ev[1], g.cur) != hipSuccess) rc = fail(OPO_ERR_HIP, "event record");
   float ms = 0;
   if (rc == OPO_OK && (hipEventSynchronize(ev[1]) != hipSuccess || hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess))
@@ -1394,18 +1563,13 @@ int engine_time_slices(Engine &E, Group &g, int iters, double *slice_us) {
 // fork and one join each group's stream runs `iters` back-to-back (column,
 // row) pairs; *slice_us is the time from the fork to the join per slice.
 int engine_time_joint(Engine &E, int iters, double *slice_us) {
-  using namespace opo;
   RCHK(sync_insts(E));
   RCHK(reset_counters(E, 0));
   auto slices = [&](int k) -> int {
     RCHK(fork_groups(E));
     int r = OPO_OK;
     for (auto &g : E.groups) {
-      const int A = all_mask(g);
-      for (int it = 0; it < k && r == OPO_OK; ++it) {
-        r = emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, 0, 1 % E.NZ, 0, 0);
-        if (r == OPO_OK) r = emit_row(E, g, false, A);
-      }
+      if (r == OPO_OK) r = time_some_slices(E, g, k);
     }
     const int j = join_groups(E);
     return r != OPO_OK ? r : j;
@@ -1804,7 +1968,9 @@ int engine_autotune(Engine &E, int iters) {
     // quarter-line column tiles and one-row row tiles: more, smaller blocks
     const bool small = (long long)n * g.N <= (1LL << 17);
     std::vector<int> cts = {ct0 / 2, ct0, ct0 * 2}, rts = {64, 128, 256, 512};
-    if (small) { cts.insert(cts.begin(), ct0 / 4); rts.insert(rts.begin(), 32); }
+    const bool res = time_resident(E);
+    if (res) { cts = {ct0}; rts = {64}; xcds = {0}; }  // its tiles follow from the samples per thread
+    else if (small) { cts.insert(cts.begin(), ct0 / 4); rts.insert(rts.begin(), 32); }
     bool can_fac = true;
     for (auto &I : g.inst) can_fac &= I.use_fac;
     std::vector<int> phases = {0};
@@ -1815,8 +1981,9 @@ int engine_autotune(Engine &E, int iters) {
       if (set_tuning(E, g, &tt) != OPO_OK) return 1;  // shape does not fit: skip
       RCHK(sync_insts(E));
       double u0 = 0, u1 = 0;
-      RCHK(engine_time_slices(E, g, iters, &u0));
-      RCHK(engine_time_slices(E, g, iters, &u1));
+      const int n = res ? std::max(iters, 16) : iters;  // (one launch for all slices: more of them outweigh its start)
+      RCHK(engine_time_slices(E, g, n, &u0));
+      RCHK(engine_time_slices(E, g, n, &u1));
       *us = std::min(u0, u1);
       return OPO_OK;
     };

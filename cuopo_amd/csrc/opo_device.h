@@ -32,6 +32,11 @@ template <> struct vec2<float> { using type = float2; };
 template <typename S> __device__ __forceinline__ __attribute__((address_space(1))) S *gp_scalar(S *p) {
   return (__attribute__((address_space(1))) S *)p;
 }
+// The same in the constant address space: data that no kernel in flight
+// writes.  Uniform reads are scalar loads even in a kernel that stores.
+template <typename S> __device__ __forceinline__ const __attribute__((address_space(4))) S *cp_scalar(const S *p) {
+  return (const __attribute__((address_space(4))) S *)p;
+}
 template <typename V> struct native2;
 template <> struct native2<double2> { using type = double __attribute__((ext_vector_type(2))); };
 template <> struct native2<float2> { using type = float __attribute__((ext_vector_type(2))); };
@@ -64,8 +69,16 @@ template <typename V> __device__ __forceinline__ V mk(decltype(V::x) a, decltype
 }
 template <typename V> __device__ __forceinline__ V cadd(V a, V b) { return mk<V>(a.x + b.x, a.y + b.y); }
 template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>(a.x - b.x, a.y - b.y); }
+// Complex product.  FP64 by explicit fused multiply-adds: every kernel that
+// runs a stage (one launch per stage, or the resident pass) then rounds alike,
+// whatever the compiler would have contracted, and their results are the same
+// bit for bit.  (FP32 contracts alike in both as written; the tests compare.)
 template <typename V> __device__ __forceinline__ V cmul(V a, V b) {
-  return mk<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  if constexpr (std::is_same<V, double2>::value) {
+    return mk<V>(__builtin_fma(-a.y, b.y, a.x * b.x), __builtin_fma(a.x, b.y, a.y * b.x));
+  } else {
+    return mk<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  }
 }
 template <typename V> __device__ __forceinline__ V cconj(V a) { return mk<V>(a.x, -a.y); }
 template <typename V> __device__ __forceinline__ V cscale(V a, decltype(V::x) s) { return mk<V>(a.x * s, a.y * s); }
@@ -269,6 +282,90 @@ __device__ __forceinline__ void load_twiddles(V *treg, int t, G g) {
       }
     }
     load_twiddles<M, E, Q + 1>(treg, t, g);
+  }
+}
+
+// ---- pointwise nonlinear half step, shared by the stage kernels ----
+
+template <typename V, typename P> __device__ __forceinline__ V ld_c(P p) {
+  return mk<V>((decltype(V::x))p[0], (decltype(V::x))p[1]);
+}
+
+// four-step twiddle e^{S 2 pi i e/N} from two small tables
+template <int S, typename V>
+__device__ __forceinline__ V twiddle_n(unsigned e, const V *__restrict__ lo, const V *__restrict__ hi, int lobits) {
+  const V w = cmul(hi[e >> lobits], lo[e & ((1u << lobits) - 1u)]);
+  return tw_sign<S>(w);
+}
+
+// Field f of three values.  The operands are taken by value so the choice is a
+// register select, never a load through a selected address (which would keep
+// the field arrays out of registers).
+template <typename V> __device__ __forceinline__ V pick(int f, V a, V b, V c) {
+  const V r = f == 1 ? b : c;
+  return f == 0 ? a : r;
+}
+
+// Coefficients of one nonlinear half step (slice s), read once per block at
+// kernel start so their latency overlaps the field loads.
+template <int NF, typename V> struct NlCoef {
+  V c[NF == 3 ? 3 : 6];
+  decltype(V::x) kp, ks, h;
+};
+
+template <int NF, typename V, typename P>
+__device__ __forceinline__ NlCoef<NF, V> load_nl_at(P q, double kp, double ks, double h) {
+  NlCoef<NF, V> r;
+#pragma unroll
+  for (int j = 0; j < (NF == 3 ? 3 : 6); ++j) r.c[j] = ld_c<V>(q + 2 * j);
+  using R = decltype(V::x);
+  r.kp = (R)kp; r.ks = (R)ks; r.h = (R)h;
+  return r;
+}
+
+template <int NF, typename V>
+__device__ __forceinline__ NlCoef<NF, V> load_nl(const double *nl, double kp, double ks, double h, int s) {
+  return load_nl_at<NF, V>(gp_scalar(nl) + 16 * s, kp, ks, h);
+}
+
+// Pointwise nonlinear half step on all fields of K samples.
+template <int NF, int K, typename V>
+__device__ __forceinline__ void nl_half_pt(V *xp, V *xs, V *xi, const NlCoef<NF, V> &q) {
+  if constexpr (NF == 3) {
+    // Closed form of cwes3.cuh:153-172: every stage evaluates dAdz on the
+    // unchanged fields, so A += (h/6)(k1+2k2+2k3+k4) = A + C*P(A) with
+    // C = i kappa (h/6)(E(z)+4E(z+dz/4)+E(z+dz/2)) precomputed in FP64.
+    const V Cp = q.c[0], Cs = q.c[1], Ci = q.c[2];
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+      const V ap = xp[m], as = xs[m], ai = xi[m];
+      xp[m] = cadd(ap, cmul(Cp, cmul(as, ai)));
+      xs[m] = cadd(as, cmul(Cs, cmul(ap, cconj(ai))));
+      xi[m] = cadd(ai, cmul(Ci, cmul(ap, cconj(as))));
+    }
+  } else {
+    // cwes2.cuh:147-166: stages 2-4 evaluate dAdz on A + s*k (s = 0.5, 0.5, 1).
+    using R = decltype(V::x);
+    const V ep0 = q.c[0], ep1 = q.c[1], ep2 = q.c[2];
+    const V em0 = q.c[3], em1 = q.c[4], em2 = q.c[5];
+    const V ikp = mk<V>((R)0, q.kp), iks = mk<V>((R)0, q.ks);
+    const R h = q.h;
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+      const V ap = xp[m], as = xs[m];
+      V k1p = cmul(cmul(cmul(ikp, as), as), ep0), k1s = cmul(cmul(cmul(iks, ap), cconj(as)), em0);
+      V bp = cadd(ap, cscale(k1p, (R)0.5)), bs = cadd(as, cscale(k1s, (R)0.5));
+      V k2p = cmul(cmul(cmul(ikp, bs), bs), ep1), k2s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
+      bp = cadd(ap, cscale(k2p, (R)0.5)); bs = cadd(as, cscale(k2s, (R)0.5));
+      V k3p = cmul(cmul(cmul(ikp, bs), bs), ep1), k3s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
+      bp = cadd(ap, k3p); bs = cadd(as, k3s);
+      V k4p = cmul(cmul(cmul(ikp, bs), bs), ep2), k4s = cmul(cmul(cmul(iks, bp), cconj(bs)), em2);
+      V sp = cadd(cadd(cadd(k1p, cscale(k2p, (R)2)), cscale(k3p, (R)2)), k4p);
+      V ss = cadd(cadd(cadd(k1s, cscale(k2s, (R)2)), cscale(k3s, (R)2)), k4s);
+      sp = cscale(sp, h); ss = cscale(ss, h);
+      xp[m] = cadd(ap, mk<V>(sp.x / (R)6, sp.y / (R)6));
+      xs[m] = cadd(as, mk<V>(ss.x / (R)6, ss.y / (R)6));
+    }
   }
 }
 

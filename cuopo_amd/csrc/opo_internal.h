@@ -13,6 +13,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 
 #include "../../include/opo.h"
 
@@ -63,6 +64,7 @@ struct OpoInst {
   void *snap;              // NF*N complex: time-domain fields at the last check
   int active_v;            // copy of *active read by the stage kernels with the other fields
   int pad_;
+  const void *lfac_spt[2]; // lfac for 8 / 4 samples per thread (the resident pass chooses its own)
 };
 
 struct ColArgs {
@@ -79,6 +81,10 @@ struct ColArgs {
   int xcd_pack;      // 1: grid is 8x wider and only blocks with blockIdx.x % 8 == 0 work
   int swz;           // 1: XCD-contiguous tile order (tiles narrower than a cache line)
   int spt;           // samples per thread of the column FFT (4 or 8)
+  // counters of the resident pass that follows (opo_resident.h), cleared by
+  // the general (boundary) kernel; null when none follows
+  unsigned long long *zero;
+  int zero_words;
   // single always-active instance (solver): the slice-interior kernel takes
   // these instead of reading the instance descriptor first
   int direct;
@@ -99,6 +105,46 @@ struct RowArgs {
   void *d_state;
   const void *d_lin, *d_lfac, *d_gdd;
 };
+
+// Resident crystal pass (opo_resident.h): counters of the XCDs' teams, each on
+// a cache line of its own, cleared before every pass.
+constexpr int kXcds = 8, kMaxTeams = 32;  // teams per XCD
+struct alignas(128) ResLine {
+  unsigned v;
+};
+struct ResTeam {
+  alignas(128) unsigned done;            // stages finished, summed over the team's blocks
+  alignas(128) unsigned long long cur;   // (turn << 32) | instance the team works on
+};
+struct ResSync {
+  ResLine next;                          // instances handed out
+  ResLine join[kXcds], size[kXcds];      // blocks that joined an XCD's teams; the count they were closed with
+  ResTeam team[kMaxTeams * kXcds];       // team-major, so the used ones are a prefix
+};
+struct ResArgs {
+  const void *tw1, *tw2, *twlo, *twhi;
+  int lobits, xl_bits;
+  int NZ, count;     // count: instances of `insts`
+  const OpoInst *insts2;  // ... then count2 of a second group of the same grid size
+  int count2;
+  int teams;         // per XCD
+  int sub;           // tiles a block works on side by side
+  int expect;        // blocks per XCD
+  int spread, prefer;  // fewer instances than teams: XCD that takes the first one
+  unsigned zero;     // 0
+  void *sync;        // ResSync
+  int *err;          // set on a time-out, never cleared by a kernel
+};
+// threads per block of the resident pass
+constexpr int res_max_threads(int, int) { return 768; }
+bool resident_supported(int N1, int N2, int ce, int re);
+int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoInst *insts, const ResArgs &a, int grid,
+                    void *stream);
+
+constexpr int kMaxDevices = 64;
+constexpr int kMaxDynLds = 159 * 1024;  // a kernel of 1 KiB or less of static LDS
+// a kernel opts in to more than 64 KiB of LDS once per device
+int opt_in_big_lds(const void *kern, std::once_flag (&flags)[kMaxDevices], int bytes = 160 * 1024);
 
 struct TickArgs {
   int count;

@@ -25,84 +25,6 @@
 
 namespace opo {
 
-template <typename V, typename P> __device__ __forceinline__ V ld_c(P p) {
-  return mk<V>((decltype(V::x))p[0], (decltype(V::x))p[1]);
-}
-
-// four-step twiddle e^{S 2 pi i e/N} from two small tables
-template <int S, typename V>
-__device__ __forceinline__ V twiddle_n(unsigned e, const V *__restrict__ lo, const V *__restrict__ hi, int lobits) {
-  const V w = cmul(hi[e >> lobits], lo[e & ((1u << lobits) - 1u)]);
-  return tw_sign<S>(w);
-}
-
-// Field f of three values.  The operands are taken by value so the choice is a
-// register select, never a load through a selected address (which would keep
-// the field arrays out of registers).
-template <typename V> __device__ __forceinline__ V pick(int f, V a, V b, V c) {
-  const V r = f == 1 ? b : c;
-  return f == 0 ? a : r;
-}
-
-// Coefficients of one nonlinear half step (slice s), read once per block at
-// kernel start so their latency overlaps the field loads.
-template <int NF, typename V> struct NlCoef {
-  V c[NF == 3 ? 3 : 6];
-  decltype(V::x) kp, ks, h;
-};
-
-template <int NF, typename V>
-__device__ __forceinline__ NlCoef<NF, V> load_nl(const double *nl, double kp, double ks, double h, int s) {
-  NlCoef<NF, V> r;
-  const auto q = gp_scalar(nl) + 16 * s;
-#pragma unroll
-  for (int j = 0; j < (NF == 3 ? 3 : 6); ++j) r.c[j] = ld_c<V>(q + 2 * j);
-  using R = decltype(V::x);
-  r.kp = (R)kp; r.ks = (R)ks; r.h = (R)h;
-  return r;
-}
-
-// Pointwise nonlinear half step on all fields of K samples.
-template <int NF, int K, typename V>
-__device__ __forceinline__ void nl_half_pt(V *xp, V *xs, V *xi, const NlCoef<NF, V> &q) {
-  if constexpr (NF == 3) {
-    // Closed form of cwes3.cuh:153-172: every stage evaluates dAdz on the
-    // unchanged fields, so A += (h/6)(k1+2k2+2k3+k4) = A + C*P(A) with
-    // C = i kappa (h/6)(E(z)+4E(z+dz/4)+E(z+dz/2)) precomputed in FP64.
-    const V Cp = q.c[0], Cs = q.c[1], Ci = q.c[2];
-#pragma unroll
-    for (int m = 0; m < K; ++m) {
-      const V ap = xp[m], as = xs[m], ai = xi[m];
-      xp[m] = cadd(ap, cmul(Cp, cmul(as, ai)));
-      xs[m] = cadd(as, cmul(Cs, cmul(ap, cconj(ai))));
-      xi[m] = cadd(ai, cmul(Ci, cmul(ap, cconj(as))));
-    }
-  } else {
-    // cwes2.cuh:147-166: stages 2-4 evaluate dAdz on A + s*k (s = 0.5, 0.5, 1).
-    using R = decltype(V::x);
-    const V ep0 = q.c[0], ep1 = q.c[1], ep2 = q.c[2];
-    const V em0 = q.c[3], em1 = q.c[4], em2 = q.c[5];
-    const V ikp = mk<V>((R)0, q.kp), iks = mk<V>((R)0, q.ks);
-    const R h = q.h;
-#pragma unroll
-    for (int m = 0; m < K; ++m) {
-      const V ap = xp[m], as = xs[m];
-      V k1p = cmul(cmul(cmul(ikp, as), as), ep0), k1s = cmul(cmul(cmul(iks, ap), cconj(as)), em0);
-      V bp = cadd(ap, cscale(k1p, (R)0.5)), bs = cadd(as, cscale(k1s, (R)0.5));
-      V k2p = cmul(cmul(cmul(ikp, bs), bs), ep1), k2s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
-      bp = cadd(ap, cscale(k2p, (R)0.5)); bs = cadd(as, cscale(k2s, (R)0.5));
-      V k3p = cmul(cmul(cmul(ikp, bs), bs), ep1), k3s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
-      bp = cadd(ap, k3p); bs = cadd(as, k3s);
-      V k4p = cmul(cmul(cmul(ikp, bs), bs), ep2), k4s = cmul(cmul(cmul(iks, bp), cconj(bs)), em2);
-      V sp = cadd(cadd(cadd(k1p, cscale(k2p, (R)2)), cscale(k3p, (R)2)), k4p);
-      V ss = cadd(cadd(cadd(k1s, cscale(k2s, (R)2)), cscale(k3s, (R)2)), k4s);
-      sp = cscale(sp, h); ss = cscale(ss, h);
-      xp[m] = cadd(ap, mk<V>(sp.x / (R)6, sp.y / (R)6));
-      xs[m] = cadd(as, mk<V>(ss.x / (R)6, ss.y / (R)6));
-    }
-  }
-}
-
 // Column stage.  The block holds CT columns of every field; the threads are
 // split into NF groups of FT = CT*N1/E (E = 4 or 8 samples per thread), and
 // group f runs field f's column FFTs, so the fields' transforms proceed on
@@ -119,6 +41,13 @@ __global__ __launch_bounds__(E == 4 ? 1024 : 512) void col_stage(const OpoInst *
   V *ltw = reinterpret_cast<V *>(smem_raw);  // N1-point root table
   V *lds = ltw + N1;                         // 2 buffers (1 for wave) x NF fields x CT*N1
 
+  if constexpr (!MID) {
+    if (a.zero) {
+      const int all = (int)(gridDim.x * gridDim.y * blockDim.x);
+      for (int i = (int)((blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x); i < a.zero_words; i += all)
+        a.zero[i] = 0;
+    }
+  }
   const OpoInst *I = insts + blockIdx.y;
   if constexpr (!DIRECT) {
     if (I->active_v == 0) return;  // block-uniform
@@ -525,15 +454,14 @@ __global__ __launch_bounds__(64) void tick_kernel(OpoInst *__restrict__ insts, T
 
 // gfx950 has 160 KiB of LDS per CU; a kernel opts in above 64 KiB once per
 // device (the attribute belongs to the device's copy of the function).
-constexpr int kMaxDevices = 64;
-static int opt_in_big_lds(const void *kern, std::once_flag (&flags)[kMaxDevices]) {
+int opt_in_big_lds(const void *kern, std::once_flag (&flags)[kMaxDevices], int bytes) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return (int)hipErrorInvalidDevice;
   // a failed opt-in leaves the flag unset (call_once does not complete when
   // its callable throws), so the next launch on this device tries again
   try {
     std::call_once(flags[dev], [&] {
-      const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
       if (e != hipSuccess) throw e;
     });
   } catch (hipError_t e) {
@@ -674,6 +602,26 @@ int launch_copy(const void *src, void *dst, long long n, void *stream, void *ev0
 int launch_tick(OpoInst *insts, const TickArgs &a, void *stream) {
   hipLaunchKernelGGL(tick_kernel, dim3(a.count), dim3(64), 0, (hipStream_t)stream, insts, a);
   return (int)hipGetLastError();
+}
+
+// ------------------------------------------------ resident crystal pass
+// One translation unit per element type and field count (opo_resident_*.hip).
+int launch_resident_f64_2(int, int, int, int, const OpoInst *, const ResArgs &, int, hipStream_t);
+int launch_resident_f64_3(int, int, int, int, const OpoInst *, const ResArgs &, int, hipStream_t);
+int launch_resident_f32_2(int, int, int, int, const OpoInst *, const ResArgs &, int, hipStream_t);
+int launch_resident_f32_3(int, int, int, int, const OpoInst *, const ResArgs &, int, hipStream_t);
+
+// N = 2^10 .. 2^15, and a row and a column of one tile fit one wavefront
+bool resident_supported(int N1, int N2, int ce, int re) {
+  const int N = N1 * N2;
+  return N >= (1 << 10) && N <= (1 << 15) && (ce == 4 || ce == 8) && N2 <= 64 * re && (re == 8 || re == 4);
+}
+
+int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoInst *insts, const ResArgs &a, int grid,
+                    void *stream) {
+  auto f = fp32 ? (NF == 3 ? launch_resident_f32_3 : launch_resident_f32_2)
+                : (NF == 3 ? launch_resident_f64_3 : launch_resident_f64_2);
+  return f(N1, N2, ce, re, insts, a, grid, (hipStream_t)stream);
 }
 
 // ------------------------------------------------ round-trip extrapolation

@@ -1,0 +1,9 @@
+// opo_resident_f32_2.hip -- the resident crystal pass, complex64 fields, two equations.
+#include "opo_resident.h"
+
+namespace opo {
+int launch_resident_f32_2(int N1, int N2, int ce, int re, const OpoInst *insts, const ResArgs &a, int grid,
+                            hipStream_t s) {
+  return launch_resident_t<float, 2>(N1, N2, ce, re, insts, a, grid, s);
+}
+}  // namespace opo
