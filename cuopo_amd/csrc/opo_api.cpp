@@ -455,10 +455,10 @@ int upload_instance(Engine &E, Group &g, int k, const double *w, const double *T
         const cd C[3] = {cd(0, p.kp) * em * h / 6.0, cd(0, p.ks) * ep * h / 6.0, cd(0, p.ki) * ep * h / 6.0};
         for (int j = 0; j < 3; ++j) { q[2 * j] = C[j].real(); q[2 * j + 1] = C[j].imag(); }
       } else {
-        // dAdz (cwes2.cuh:37-38): pump e^{+i dk z}, signal e^{-i dk z}
+        // dAdz (cwes2.cuh:37-38): pump i kappa_p e^{+i dk z}, signal i kappa_s e^{-i dk z}
         const double zs[3] = {za, zb, zc};
         for (int j = 0; j < 3; ++j) {
-          const cd a = ex(+p.dk * zs[j]), b = ex(-p.dk * zs[j]);
+          const cd a = cd(0, p.kp) * ex(+p.dk * zs[j]), b = cd(0, p.ks) * ex(-p.dk * zs[j]);
           q[2 * j] = a.real(); q[2 * j + 1] = a.imag();
           q[6 + 2 * j] = b.real(); q[6 + 2 * j + 1] = b.imag();
         }
@@ -508,8 +508,7 @@ OpoInst make_desc(const Engine &E, const Group &g, int k) {
   d.save_slots = p.regime == OPO_CW ? p.Nrts : p.NRT;
   d.nrt = p.NRT;
   d.regime = p.regime;
-  d.h = p.dz / 2;
-  d.kp = p.kp; d.ks = p.ks; d.ki = p.ki;
+  d.h6 = p.dz / 2 / 6;
   d.sqrt_rs = std::sqrt(p.Rs); d.sqrt_ri = std::sqrt(p.Ri);  // AddPhase, functions.cuh:145
   d.mir[0] = std::cos(kPi * p.delta); d.mir[1] = std::sin(kPi * p.delta);
   d.rt = g.d_rt + k; d.active = g.d_active + k; d.partials = g.d_partials + (size_t)k * g.N2;
@@ -676,7 +675,7 @@ int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int 
     const Instance &I = g.inst[0];
     a.direct = 1;
     a.d_state = I.state; a.d_nl = I.nl;
-    a.d_kp = I.prm.kp; a.d_ks = I.prm.ks; a.d_h = I.prm.dz / 2;
+    a.d_h6 = I.prm.dz / 2 / 6;
   }
   const int threads_ct = g.ct;
   int e = opo::launch_col(g.fp32, g.N1, g.NF, threads_ct, g.launch_n, g.d_insts, a, g.cur, e0, e1);

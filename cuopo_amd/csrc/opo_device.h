@@ -73,9 +73,11 @@ template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>
 // runs a stage (one launch per stage, or the resident pass) then rounds alike,
 // whatever the compiler would have contracted, and their results are the same
 // bit for bit.  (FP32 contracts alike in both as written; the tests compare.)
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <typename V> __device__ __forceinline__ V cmul(V a, V b) {
   if constexpr (std::is_same<V, double2>::value) {
-    return mk<V>(__builtin_fma(-a.y, b.y, a.x * b.x), __builtin_fma(a.x, b.y, a.y * b.x));
+    return mk<V>(fma_(-a.y, b.y, a.x * b.x), fma_(a.x, b.y, a.y * b.x));
   } else {
     return mk<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
   }
@@ -307,25 +309,24 @@ template <typename V> __device__ __forceinline__ V pick(int f, V a, V b, V c) {
 }
 
 // Coefficients of one nonlinear half step (slice s), read once per block at
-// kernel start so their latency overlaps the field loads.
+// kernel start so their latency overlaps the field loads.  Three equations:
+// the closed form's three; two: i kappa e^{+-i dk z} at the three stage
+// positions, pump then signal, and h6 = (dz/2)/6.
 template <int NF, typename V> struct NlCoef {
   V c[NF == 3 ? 3 : 6];
-  decltype(V::x) kp, ks, h;
+  decltype(V::x) h6;
 };
 
-template <int NF, typename V, typename P>
-__device__ __forceinline__ NlCoef<NF, V> load_nl_at(P q, double kp, double ks, double h) {
+template <int NF, typename V, typename P> __device__ __forceinline__ NlCoef<NF, V> load_nl_at(P q, double h6) {
   NlCoef<NF, V> r;
 #pragma unroll
   for (int j = 0; j < (NF == 3 ? 3 : 6); ++j) r.c[j] = ld_c<V>(q + 2 * j);
-  using R = decltype(V::x);
-  r.kp = (R)kp; r.ks = (R)ks; r.h = (R)h;
+  r.h6 = (decltype(V::x))h6;
   return r;
 }
 
-template <int NF, typename V>
-__device__ __forceinline__ NlCoef<NF, V> load_nl(const double *nl, double kp, double ks, double h, int s) {
-  return load_nl_at<NF, V>(gp_scalar(nl) + 16 * s, kp, ks, h);
+template <int NF, typename V> __device__ __forceinline__ NlCoef<NF, V> load_nl(const double *nl, double h6, int s) {
+  return load_nl_at<NF, V>(gp_scalar(nl) + 16 * s, h6);
 }
 
 // Pointwise nonlinear half step on all fields of K samples.
@@ -345,26 +346,25 @@ __device__ __forceinline__ void nl_half_pt(V *xp, V *xs, V *xi, const NlCoef<NF,
     }
   } else {
     // cwes2.cuh:147-166: stages 2-4 evaluate dAdz on A + s*k (s = 0.5, 0.5, 1).
+    // With kappa and the phase in one coefficient and h/6 in one factor a half
+    // step is 92 instructions per sample; with kappa, the phase, h and the
+    // division by 6 each by itself it was about 170, more than the transforms
+    // around it (one 2^12 instance, FP64: 8.15 us per slice then, 6.38 now; launch by launch 10.3, 8.95).
     using R = decltype(V::x);
-    const V ep0 = q.c[0], ep1 = q.c[1], ep2 = q.c[2];
-    const V em0 = q.c[3], em1 = q.c[4], em2 = q.c[5];
-    const V ikp = mk<V>((R)0, q.kp), iks = mk<V>((R)0, q.ks);
-    const R h = q.h;
+    const V *cp = q.c, *cs = q.c + 3;
+    auto madd = [](R s, V k, V x) { return mk<V>(fma_(s, k.x, x.x), fma_(s, k.y, x.y)); };
 #pragma unroll
     for (int m = 0; m < K; ++m) {
       const V ap = xp[m], as = xs[m];
-      V k1p = cmul(cmul(cmul(ikp, as), as), ep0), k1s = cmul(cmul(cmul(iks, ap), cconj(as)), em0);
-      V bp = cadd(ap, cscale(k1p, (R)0.5)), bs = cadd(as, cscale(k1s, (R)0.5));
-      V k2p = cmul(cmul(cmul(ikp, bs), bs), ep1), k2s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
-      bp = cadd(ap, cscale(k2p, (R)0.5)); bs = cadd(as, cscale(k2s, (R)0.5));
-      V k3p = cmul(cmul(cmul(ikp, bs), bs), ep1), k3s = cmul(cmul(cmul(iks, bp), cconj(bs)), em1);
+      const V k1p = cmul(cp[0], cmul(as, as)), k1s = cmul(cs[0], cmul(ap, cconj(as)));
+      V bp = madd((R)0.5, k1p, ap), bs = madd((R)0.5, k1s, as);
+      const V k2p = cmul(cp[1], cmul(bs, bs)), k2s = cmul(cs[1], cmul(bp, cconj(bs)));
+      bp = madd((R)0.5, k2p, ap); bs = madd((R)0.5, k2s, as);
+      const V k3p = cmul(cp[1], cmul(bs, bs)), k3s = cmul(cs[1], cmul(bp, cconj(bs)));
       bp = cadd(ap, k3p); bs = cadd(as, k3s);
-      V k4p = cmul(cmul(cmul(ikp, bs), bs), ep2), k4s = cmul(cmul(cmul(iks, bp), cconj(bs)), em2);
-      V sp = cadd(cadd(cadd(k1p, cscale(k2p, (R)2)), cscale(k3p, (R)2)), k4p);
-      V ss = cadd(cadd(cadd(k1s, cscale(k2s, (R)2)), cscale(k3s, (R)2)), k4s);
-      sp = cscale(sp, h); ss = cscale(ss, h);
-      xp[m] = cadd(ap, mk<V>(sp.x / (R)6, sp.y / (R)6));
-      xs[m] = cadd(as, mk<V>(ss.x / (R)6, ss.y / (R)6));
+      const V k4p = cmul(cp[2], cmul(bs, bs)), k4s = cmul(cs[2], cmul(bp, cconj(bs)));
+      xp[m] = madd(q.h6, madd((R)2, cadd(k2p, k3p), cadd(k1p, k4p)), ap);
+      xs[m] = madd(q.h6, madd((R)2, cadd(k2s, k3s), cadd(k1s, k4s)), as);
     }
   }
 }

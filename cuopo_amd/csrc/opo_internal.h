@@ -39,7 +39,7 @@ struct OpoInst {
                            // Z (E*N1), S (N2), Xhi (N/E >> L), Xlo (2^L); or null
   const void *gdd;         // 2N complex (signal, idler): e^{i w^2 GDD/2}/N, permuted; null if unused
   const void *eom;         // N complex: e^{i m sin(2 pi fpm T)}, time order; null if unused
-  const double *nl;        // NZ*16 doubles: 8 complex FP64 coefficients per slice
+  const double *nl;        // NZ*16 doubles: 8 complex FP64 coefficients per slice (see NlCoef)
   const void *pump;        // pump_len complex (Ap_in)
   long long pump_len;
   void *save[3];           // pump, signal, idler save buffers (slots*N complex) or null
@@ -47,8 +47,7 @@ struct OpoInst {
   int save_slots;
   int nrt;                 // NRT (NS slot arithmetic)
   int regime;              // 0 CW, 1 NS
-  double h;                // dz/2, the RK step of the two-equation chain
-  double kp, ks, ki;       // kappas (two-equation chain)
+  double h6;               // (dz/2)/6, the RK weight of the two-equation chain
   double sqrt_rs, sqrt_ri; // mirror amplitude factors
   double mir[2];           // e^{i pi delta}
   int *rt;                 // round-trip counter
@@ -90,7 +89,7 @@ struct ColArgs {
   int direct;
   void *d_state;
   const double *d_nl;
-  double d_kp, d_ks, d_h;
+  double d_h6;
 };
 
 struct RowArgs {

@@ -119,11 +119,11 @@ __global__ __launch_bounds__(E == 4 ? 1024 : 512) void col_stage(const OpoInst *
   __builtin_amdgcn_sched_barrier(0);
   NlCoef<NF, V> nle{}, nls{};
   if constexpr (DIRECT) {
-    nle = load_nl<NF, V>(a.d_nl, a.d_kp, a.d_ks, a.d_h, a.s_end);
-    nls = load_nl<NF, V>(a.d_nl, a.d_kp, a.d_ks, a.d_h, a.s_start);
+    nle = load_nl<NF, V>(a.d_nl, a.d_h6, a.s_end);
+    nls = load_nl<NF, V>(a.d_nl, a.d_h6, a.s_start);
   } else {
-    if (ops & OP_NL_END) nle = load_nl<NF, V>(I->nl, I->kp, I->ks, I->h, a.s_end);
-    if (ops & OP_NL_START) nls = load_nl<NF, V>(I->nl, I->kp, I->ks, I->h, a.s_start);
+    if (ops & OP_NL_END) nle = load_nl<NF, V>(I->nl, I->h6, a.s_end);
+    if (ops & OP_NL_START) nls = load_nl<NF, V>(I->nl, I->h6, a.s_start);
   }
   V W[E];
   V x0r{}, b1r{};  // FP64: the four-step roots' base, kept across the pointwise program instead of W

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
     const auto lfac = gp(reinterpret_cast<const V *>(I->lfac_spt[ER == 8 ? 0 : 1]));
     const auto lin = gp(reinterpret_cast<const V *>(I->lin));
     const double *nl = I->nl;
-    const double kp = I->kp, ks = I->ks, hh = I->h;
+    const double h6 = I->h6;
     bool first = true;
 
     // Waits until every block of the team has finished the stage before.
@@ -281,8 +281,8 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
       {
         const int l = opaque(lane);
         const int c = l & (CT - 1), t = l / CT;
-        const NlCoef<NF, V> nle = load_nl_at<NF, V>(cp_scalar(nl) + 16 * s, kp, ks, hh);
-        const NlCoef<NF, V> nls = load_nl_at<NF, V>(cp_scalar(nl) + 16 * (s + 1), kp, ks, hh);
+        const NlCoef<NF, V> nle = load_nl_at<NF, V>(cp_scalar(nl) + 16 * s, h6);
+        const NlCoef<NF, V> nls = load_nl_at<NF, V>(cp_scalar(nl) + 16 * (s + 1), h6);
         constexpr int fstride = 64 * EC;
         bool waited = false;
         for (int t0 = 0; t0 < NTC; t0 += workers) {
