@@ -2,8 +2,9 @@
 // GELU -> n_out) trained and evaluated on the GPU with BF16 weights and
 // activations and FP32 accumulation.  Every matrix product (forward, weight
 // gradient, input gradient) runs through one hand-written MFMA kernel
-// (v_mfma_f32_16x16x16_bf16, 64x64 block tiles); bias/GELU/GELU' are fused into
-// its epilogue.  FP32 master weights, Adam in FP32.  No reference
+// (v_mfma_f32_16x16x16_bf16, 64x64 or 32x32 block tiles); bias/GELU/GELU' are
+// fused into its epilogue and the bias gradients' column sums run beside the
+// weight gradients.  FP32 master weights, Adam in FP32.  No reference
 // counterpart: cuOPO has no learned component.
 #include <hip/hip_runtime.h>
 
@@ -49,13 +50,6 @@ __host__ __device__ inline unsigned short f2bf(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return (unsigned short)(u >> 16);
 }
-__host__ __device__ inline float bf2f(unsigned short h) {
-  unsigned int u = (unsigned int)h << 16;
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
-}
-
 __device__ inline float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 __device__ inline float gelu_grad(float x) {
   return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
@@ -68,76 +62,220 @@ enum Epi : int {
   EPI_GELU_GRAD = 3,   // C = acc * gelu'(Zprev[m, n]) (fp32)
 };
 
-// Element (r, c) of a matrix stored with row stride sr and column stride sc.
-template <typename T> __device__ inline float ldv(const T *p, long long i);
-template <> __device__ inline float ldv<float>(const float *p, long long i) { return p[i]; }
-template <> __device__ inline float ldv<unsigned short>(const unsigned short *p, long long i) { return bf2f(p[i]); }
+// One operand of a product: R rows (A's m or B's n) of K values.  `kc`: the K
+// values of a row are contiguous, element (r, k) at p[r * ld + k]; otherwise
+// the rows are, at p[k * ld + r].
+template <typename T> struct Operand {
+  const T *p;
+  long long ld;
+  int R;
+  int vec;  // rows (kc) or columns (!kc) start on a vector boundary: whole vectors load at once
+};
 
 struct GemmArgs {
   int M, N, K;
-  long long a_sm, a_sk;  // A(m, k) = A[m*a_sm + k*a_sk]
-  long long b_sk, b_sn;  // B(k, n) = B[k*b_sk + n*b_sn]
   long long ldc;         // C(m, n) = C[m*ldc + n]
   const float *bias;     // [N]
   const float *zprev;    // EPI_GELU_GRAD: Z of the layer below, same shape as C
   float *zout;           // EPI_BIAS_GELU: pre-activation out (may be null)
   unsigned short *hout;  // EPI_BIAS_GELU: bf16 activation out
   float *cout;           // fp32 out
-  int epi;
+  const float *col_in;   // column sums beside the product (bias gradient), or null
+  float *col_out;        // col_out[c] = sum over r of col_in[r*cols + c], r < rows, in order
+  int col_rows, col_cols;
 };
 
-// C[M x N] = A[M x K] * B[K x N]: 256 threads, 64 x 64 tile, each wave a 32 x 32
-// quarter as 2 x 2 MFMA 16x16x16 blocks; K in steps of 16 through LDS.
-// Operand lanes of v_mfma_f32_16x16x16_bf16: lane l carries A(l%16, 4(l/16)+q)
-// and B(4(l/16)+q, l%16), q = 0..3; result register q holds D(4(l/16)+q, l%16).
-template <typename TA, typename TB>
-__global__ __launch_bounds__(256) void gemm_bf16(const TA *__restrict__ A, const TB *__restrict__ B, GemmArgs g) {
-  __shared__ unsigned short As[64][16 + 2];
-  __shared__ unsigned short Bs[16][64 + 2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int m_base = blockIdx.y * 64, n_base = blockIdx.x * 64;
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < g.K; k0 += 16) {
-    for (int e = tid; e < 64 * 16; e += 256) {
-      const int r = e / 16, kk = e % 16;  // A tile (64 x 16)
-      const int m = m_base + r, k = k0 + kk;
-      float v = (m < g.M && k < g.K) ? ldv(A, (long long)m * g.a_sm + (long long)k * g.a_sk) : 0.f;
-      As[r][kk] = f2bf(v);
-      const int kb = e / 64, c = e % 64;  // B tile (16 x 64)
-      const int kB = k0 + kb, n = n_base + c;
-      float u = (kB < g.K && n < g.N) ? ldv(B, (long long)kB * g.b_sk + (long long)n * g.b_sn) : 0.f;
-      Bs[kb][c] = f2bf(u);
-    }
-    __syncthreads();
-    bf16x4 a[2], b[2];
-    for (int i = 0; i < 2; ++i) {
-      const int r = wm * 32 + i * 16 + (lane & 15);
-      for (int q = 0; q < 4; ++q) a[i][q] = (short)As[r][4 * (lane >> 4) + q];
-    }
-    for (int j = 0; j < 2; ++j) {
-      const int c = wn * 32 + j * 16 + (lane & 15);
-      for (int q = 0; q < 4; ++q) b[j][q] = (short)Bs[4 * (lane >> 4) + q][c];
-    }
-    for (int i = 0; i < 2; ++i)
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+// A block's stage of one operand: ROWS rows x KC values, read from memory into
+// registers (fetch), then written to LDS as bf16 with K contiguous (put), so
+// that the next stages' reads are in flight while this one is multiplied.  The
+// registers hold the words as loaded: taking them apart in fetch would wait
+// for the loads there (78 instead of 40 us for 256 x 256 over K = 4096).
+template <typename T, bool KCONT, int ROWS, int KC> struct Stage {
+  // K contiguous: vectors of 8 values of a row.  Rows contiguous: 4 rows x 2
+  // values, so that pairs of K go to LDS as one word.
+  static constexpr int kUnits = ROWS * KC / 8 / 256;
+  static constexpr int kPer = 4 / sizeof(T);  // values per word
+  static constexpr int kWords = 8 / kPer;
+  static_assert(kUnits >= 1 && ROWS * KC % 2048 == 0, "whole units per thread");
+  unsigned w[kUnits][kWords];
+
+  // value j of a unit as bf16 bits
+  __device__ __forceinline__ unsigned bits(int u, int j) const {
+    if constexpr (kPer == 1) return f2bf(__builtin_bit_cast(float, w[u][j]));
+    else return j & 1 ? w[u][j / 2] >> 16 : w[u][j / 2] & 0xffffu;
   }
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
+  static __device__ __forceinline__ unsigned word(const T *q, bool on0, bool on1) {
+    if constexpr (kPer == 1) return on0 ? __builtin_bit_cast(unsigned, (float)q[0]) : 0u;
+    else return (on0 ? (unsigned)q[0] : 0u) | (on1 ? (unsigned)q[1] << 16 : 0u);
+  }
+  __device__ __forceinline__ void fetch(const Operand<T> &o, int r0, int k0, int K, int tid) {
+    struct alignas(16) Vec { unsigned x[4]; };
+    struct alignas(4 * sizeof(T)) Quad { unsigned x[4 / kPer]; };
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      const int id = tid + u * 256;
+      if constexpr (KCONT) {
+        const int r = r0 + id / (KC / 8), k = k0 + id % (KC / 8) * 8;
+        const T *q = o.p + (long long)r * o.ld + k;
+        if (o.vec && r < o.R && k + 8 <= K) {
+#pragma unroll
+          for (int j = 0; j < kWords; j += 4) {
+            const Vec h = reinterpret_cast<const Vec *>(q)[j / 4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[u][j + i] = h.x[i];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < kWords; ++j)
+            w[u][j] = word(q + j * kPer, r < o.R && k + j * kPer < K, r < o.R && k + j * kPer + 1 < K);
+        }
+      } else {
+        const int r = r0 + id % (ROWS / 4) * 4, k = k0 + id / (ROWS / 4) * 2;
+        constexpr int H = kWords / 2;  // words per k
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const T *q = o.p + (long long)(k + j) * o.ld + r;
+          if (o.vec && r + 4 <= o.R && k + j < K) {
+            const Quad h = *reinterpret_cast<const Quad *>(q);
+#pragma unroll
+            for (int i = 0; i < H; ++i) w[u][H * j + i] = h.x[i];
+          } else {
+#pragma unroll
+            for (int i = 0; i < H; ++i)
+              w[u][H * j + i] = word(q + i * kPer, k + j < K && r + i * kPer < o.R, k + j < K && r + i * kPer + 1 < o.R);
+          }
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void put(unsigned short (*lds)[KC + 8], int tid) const {
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      const int id = tid + u * 256;
+      if constexpr (KCONT) {
+        struct alignas(16) Oct { unsigned x[4]; } h;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h.x[j] = kPer == 2 ? w[u][j % kWords] : bits(u, 2 * j) | bits(u, 2 * j + 1) << 16;
+        *reinterpret_cast<Oct *>(&lds[id / (KC / 8)][id % (KC / 8) * 8]) = h;
+      } else {
+        const int r = id % (ROWS / 4) * 4, k = id / (ROWS / 4) * 2;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<unsigned *>(&lds[r + i][k]) = bits(u, i) | bits(u, 4 + i) << 16;
+      }
+    }
+  }
+};
+
+// db[c] = sum over the batch, one column per thread, in batch order; 32 rows
+// are read ahead of the sums.
+__device__ __forceinline__ void column_sums(const GemmArgs &g, int block, int tid) {
+  const int c = block * 256 + tid;
+  if (c >= g.col_cols) return;
+  float s = 0;
+  for (int r = 0; r < g.col_rows; r += 32) {
+    float z[32];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) z[j] = r + j < g.col_rows ? g.col_in[(long long)(r + j) * g.col_cols + c] : 0.f;
+#pragma unroll
+    for (int j = 0; j < 32; ++j)
+      if (r + j < g.col_rows) s += z[j];
+  }
+  g.col_out[c] = s;
+}
+
+// C[M x N] = A B^T over K: 256 threads, TILE x TILE of C, each wave a quarter
+// in 16 x 16 blocks of v_mfma_f32_16x16x16_bf16, K in stages of KC through two
+// LDS buffers (one barrier per stage) with the next stage in registers.  The
+// products are accumulated in K order, 16 at a time, whatever the tile, so a
+// result depends on neither TILE nor KC.
+// What bounds it: latency.  The network's products are 256 wide, so a launch
+// is 64-256 blocks of a few stages, and the gradient through the output layer
+// (K = 4096 for 256 x 256 results) one chain of stages per block.  Hence wide
+// loads, a stage in flight, and small tiles where 64 x 64 would leave CUs idle.
+// Measured at batch 256, width 256, 4096 outputs (us per launch), against
+// single-value loads in stages of 16 and bias sums by themselves: hidden layer
+// 27.7 -> 5.3, output layer 31.5 -> 7.5, its weight and bias gradient 34.6 +
+// 59.7 -> 13.9, the seven other 256-wide gradient products of a training step
+// 844 + 4 x 56.7 -> 90 in all, 40 of them the one over K = 4096.
+// Operand lanes: lane l carries A(l%16, 4(l/16)+q) and B(l%16, 4(l/16)+q),
+// q = 0..3; result register q holds C(4(l/16)+q, l%16).
+template <int EPI, typename TA, bool AK, typename TB, bool BK, int TILE, int KC, int AHEAD>
+__global__ __launch_bounds__(256) void gemm_bf16(Operand<TA> A, Operand<TB> B, GemmArgs g) {
+  constexpr int W = TILE / 32;  // 16 x 16 blocks per wave and direction
+  __shared__ __align__(16) unsigned short As[2][TILE][KC + 8], Bs[2][TILE][KC + 8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tiles = (g.N + TILE - 1) / TILE * ((g.M + TILE - 1) / TILE);
+  if ((int)blockIdx.x >= tiles) {  // the blocks after the product's sum the columns
+    column_sums(g, blockIdx.x - tiles, tid);
+    return;
+  }
+  const int nt = (g.N + TILE - 1) / TILE;
+  const int m_base = (int)blockIdx.x / nt * TILE, n_base = (int)blockIdx.x % nt * TILE;
+  const int wm = (wave >> 1) * (TILE / 2), wn = (wave & 1) * (TILE / 2);
+  Stage<TA, AK, TILE, KC> sa[AHEAD];
+  Stage<TB, BK, TILE, KC> sb[AHEAD];
+  f32x4 acc[W][W];
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) {
+    if (d * KC < g.K) {
+      sa[d].fetch(A, m_base, d * KC, g.K, tid);
+      sb[d].fetch(B, n_base, d * KC, g.K, tid);
+    }
+  }
+  int buf = 0;
+  for (int kd = 0; kd < g.K; kd += AHEAD * KC) {
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) {  // (d is a constant: the stages stay in registers)
+      const int k0 = kd + d * KC;
+      if (k0 >= g.K) break;
+      sa[d].put(As[buf], tid);
+      sb[d].put(Bs[buf], tid);
+      if (k0 + AHEAD * KC < g.K) {
+        sa[d].fetch(A, m_base, k0 + AHEAD * KC, g.K, tid);
+        sb[d].fetch(B, n_base, k0 + AHEAD * KC, g.K, tid);
+      }
+      __syncthreads();  // (the other buffer is rewritten only after the next stage's barrier)
+#pragma unroll
+      for (int kk = 0; kk < KC; kk += 16) {
+        if (k0 + kk < g.K) {
+          bf16x4 a[W], b[W];
+#pragma unroll
+          for (int i = 0; i < W; ++i)
+            a[i] = *reinterpret_cast<const bf16x4 *>(&As[buf][wm + 16 * i + (lane & 15)][kk + 4 * (lane >> 4)]);
+#pragma unroll
+          for (int j = 0; j < W; ++j)
+            b[j] = *reinterpret_cast<const bf16x4 *>(&Bs[buf][wn + 16 * j + (lane & 15)][kk + 4 * (lane >> 4)]);
+#pragma unroll
+          for (int i = 0; i < W; ++i)
+#pragma unroll
+            for (int j = 0; j < W; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+      }
+      buf ^= 1;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+#pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m_base + wm * 32 + i * 16 + 4 * (lane >> 4) + q;
-        const int n = n_base + wn * 32 + j * 16 + (lane & 15);
+        const int m = m_base + wm + 16 * i + 4 * (lane >> 4) + q;
+        const int n = n_base + wn + 16 * j + (lane & 15);
         if (m >= g.M || n >= g.N) continue;
         const long long o = (long long)m * g.ldc + n;
-        float v = acc[i][j][q];
-        if (g.epi == EPI_STORE) {
+        const float v = acc[i][j][q];
+        if constexpr (EPI == EPI_STORE) {
           g.cout[o] = v;
-        } else if (g.epi == EPI_BIAS) {
+        } else if constexpr (EPI == EPI_BIAS) {
           g.cout[o] = v + g.bias[n];
-        } else if (g.epi == EPI_BIAS_GELU) {
+        } else if constexpr (EPI == EPI_BIAS_GELU) {
           const float z = v + g.bias[n];
           if (g.zout) g.zout[o] = z;
           g.hout[o] = f2bf(gelu(z));
@@ -148,7 +286,8 @@ __global__ __launch_bounds__(256) void gemm_bf16(const TA *__restrict__ A, const
 }
 
 // dY = 2 (Y - T) / (B * n_out); per-block partial sums of (Y - T)^2
-__global__ void mse_grad(const float *Y, const float *T, float *dY, float *partial, long long n, float scale) {
+__global__ void mse_grad(const float *__restrict__ Y, const float *__restrict__ T, float *__restrict__ dY,
+                         float *__restrict__ partial, long long n, float scale) {
   __shared__ float red[256];
   float s = 0;
   for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
@@ -163,15 +302,6 @@ __global__ void mse_grad(const float *Y, const float *T, float *dY, float *parti
     __syncthreads();
   }
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// db[n] = sum_b dZ[b, n]
-__global__ void bias_grad(const float *dZ, float *db, int Bn, int N) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0;
-  for (int b = 0; b < Bn; ++b) s += dZ[(long long)b * N + n];
-  db[n] = s;
 }
 
 __global__ void adam_step(float *w, unsigned short *wbf, const float *gr, float *m, float *v, long long n, float lr,
@@ -225,11 +355,25 @@ int malloc_m(opo_mlp *M, void **p, size_t bytes) {
   return OPO_OK;
 }
 
-template <typename TA, typename TB>
-int gemm(opo_mlp *M, const TA *A, const TB *B, GemmArgs g) {
+// 16-byte vectors along K, or four rows at a time
+template <typename T> Operand<T> operand(const T *p, long long ld, int rows, bool kcont) {
+  const size_t step = kcont ? 16 : 4 * sizeof(T);
+  return {p, ld, rows, reinterpret_cast<uintptr_t>(p) % step == 0 && (size_t)ld * sizeof(T) % step == 0};
+}
+
+// Tiles of 64 where they fill the 256 CUs, else of 32 (four times the blocks:
+// the 256 x 256 products of the hidden layers are 64 blocks then, not 16).
+template <int EPI, bool AK, bool BK, typename TA, typename TB>
+int gemm(opo_mlp *M, const TA *A, long long lda, const TB *B, long long ldb, const GemmArgs &g) {
   if (g.M <= 0 || g.N <= 0 || g.K <= 0) return mfail(OPO_ERR_INVALID, "empty gemm");
-  dim3 grid((g.N + 63) / 64, (g.M + 63) / 64);
-  hipLaunchKernelGGL((gemm_bf16<TA, TB>), grid, dim3(256), 0, M->stream, A, B, g);
+  const Operand<TA> a = operand(A, lda, g.M, AK);
+  const Operand<TB> b = operand(B, ldb, g.N, BK);
+  const int cols = g.col_in ? (g.col_cols + 255) / 256 : 0;
+  auto tiles = [&](int t) { return (g.M + t - 1) / t * ((g.N + t - 1) / t); };
+  if (tiles(64) >= 256)
+    hipLaunchKernelGGL((gemm_bf16<EPI, TA, AK, TB, BK, 64, 64, 1>), dim3(tiles(64) + cols), dim3(256), 0, M->stream, a, b, g);
+  else
+    hipLaunchKernelGGL((gemm_bf16<EPI, TA, AK, TB, BK, 32, 128, 2>), dim3(tiles(32) + cols), dim3(256), 0, M->stream, a, b, g);
   MCHK(hipGetLastError());
   return OPO_OK;
 }
@@ -239,22 +383,18 @@ int forward(opo_mlp *M, int Bn, bool store_z) {
   const unsigned short *in = M->x_bf;
   for (int l = 0; l < M->nl; ++l) {
     GemmArgs g{};
-    g.M = Bn; g.N = M->dout[l]; g.K = M->din[l];
-    g.a_sm = M->din[l]; g.a_sk = 1;        // activations [B x din]
-    g.b_sk = 1; g.b_sn = M->din[l];        // W^T: W is [dout x din]
+    g.M = Bn; g.N = M->dout[l]; g.K = M->din[l];  // activations [B x din], W [dout x din]
     g.ldc = M->dout[l];
     g.bias = M->w + M->boff[l];
     const unsigned short *W = M->wbf + M->woff[l];
     if (l < M->nl - 1) {
-      g.epi = EPI_BIAS_GELU;
       g.zout = store_z ? M->Z[l] : nullptr;
       g.hout = M->H[l];
-      MRCHK(gemm(M, in, W, g));
+      MRCHK((gemm<EPI_BIAS_GELU, true, true>(M, in, M->din[l], W, M->din[l], g)));
       in = M->H[l];
     } else {
-      g.epi = EPI_BIAS;
       g.cout = M->Y;
-      MRCHK(gemm(M, in, W, g));
+      MRCHK((gemm<EPI_BIAS, true, true>(M, in, M->din[l], W, M->din[l], g)));
     }
   }
   return OPO_OK;
@@ -270,29 +410,22 @@ int backward(opo_mlp *M, int Bn, float *loss) {
   float *dZ = M->dA, *dNext = M->dB;
   for (int l = M->nl - 1; l >= 0; --l) {
     const unsigned short *Hin = l == 0 ? M->x_bf : M->H[l - 1];
-    // dW_l = dZ^T (B x dout -> dout x B) * Hin (B x din)
+    // dW_l = dZ^T (B x dout -> dout x B) * Hin (B x din), and db_l beside it
     GemmArgs gw{};
     gw.M = M->dout[l]; gw.N = M->din[l]; gw.K = Bn;
-    gw.a_sm = 1; gw.a_sk = M->dout[l];
-    gw.b_sk = M->din[l]; gw.b_sn = 1;
     gw.ldc = M->din[l];
-    gw.epi = EPI_STORE;
     gw.cout = M->g + M->woff[l];
-    MRCHK(gemm(M, dZ, Hin, gw));
-    hipLaunchKernelGGL(bias_grad, dim3((M->dout[l] + 255) / 256), dim3(256), 0, M->stream, dZ, M->g + M->boff[l], Bn,
-                       M->dout[l]);
-    MCHK(hipGetLastError());
+    gw.col_in = dZ; gw.col_out = M->g + M->boff[l];
+    gw.col_rows = Bn; gw.col_cols = M->dout[l];
+    MRCHK((gemm<EPI_STORE, false, false>(M, dZ, M->dout[l], Hin, M->din[l], gw)));
     if (l == 0) break;
     // dZ_{l-1} = (dZ * W_l) .* gelu'(Z_{l-1});  dZ [B x dout], W [dout x din]
     GemmArgs gh{};
     gh.M = Bn; gh.N = M->din[l]; gh.K = M->dout[l];
-    gh.a_sm = M->dout[l]; gh.a_sk = 1;
-    gh.b_sk = M->din[l]; gh.b_sn = 1;
     gh.ldc = M->din[l];
-    gh.epi = EPI_GELU_GRAD;
     gh.zprev = M->Z[l - 1];
     gh.cout = dNext;
-    MRCHK(gemm(M, dZ, M->wbf + M->woff[l], gh));
+    MRCHK((gemm<EPI_GELU_GRAD, true, false>(M, dZ, M->dout[l], M->wbf + M->woff[l], M->din[l], gh)));
     std::swap(dZ, dNext);
   }
   std::vector<float> part(nb);

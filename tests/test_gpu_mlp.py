@@ -74,3 +74,24 @@ def test_mlp_closes_on_leaving_a_with_block(gpu):
         y = net.forward(np.zeros((8, 5), np.float32))
         assert np.isfinite(y).all()
     assert net._h is None
+
+
+@pytest.mark.parametrize("shape,batch", [((3, 7, 2, 11), 5), ((9, 33, 3, 129), 200), ((5, 256, 1, 4096), 1),
+                                         ((16, 128, 2, 256), 130), ((8, 64, 1, 1000), 256), ((5, 512, 1, 8), 64)])
+def test_products_at_tile_edges(gpu, shape, batch):
+    """Both tiles, whole-vector and single-value loads (widths that are no multiple of 4 or 8), one row,
+    remainders of rows and of K.  The operands are rounded to bf16 (2^-8 relative) on both sides and the sums
+    kept in FP32, so the outputs differ by rounding flips of hidden activations: 2^-8 of an entry over
+    sqrt(width) and more of them, below 5e-3 of the whole; gradients pass twice as many: 3e-2."""
+    net, theta, rng = make(shape, batch, 4)
+    x = rng.uniform(-1, 1, (batch, shape[0])).astype(np.float32)
+    t = rng.standard_normal((batch, shape[3])).astype(np.float32)
+    ref, _, _ = M.forward(theta, shape, x, quantize=True)
+    assert rel(net.forward(x), ref) < 5e-3
+    loss, g = net.gradients(x, t)
+    rloss, rg = M.loss_and_grad(theta, shape, x, t, quantize=True)
+    assert loss == pytest.approx(rloss, rel=1e-3)
+    assert rel(g, rg) < 3e-2
+    din, dout, offs, _ = M.layers(*shape)
+    for (wo, bo), a, b in zip(offs, din, dout):
+        assert rel(g[bo:bo + b], rg[bo:bo + b]) < 5e-2
