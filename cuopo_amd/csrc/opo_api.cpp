@@ -136,6 +136,7 @@ struct Engine {
   int accel_every = 0;     // round-trip extrapolation every this many round trips (0: off), see accel_step
   int accel_start = 1000;  // ... from this many round trips of the run on
   bool resident = true;  // crystal passes as one launch where every group allows it (opo_resident.h)
+  bool timing = false;   // the autotuner is timing slices
   bool forked = false;   // the groups' chains run on their own streams (fork_groups .. join_groups)
   bool save_enabled = false;
   hipGraphExec_t gexec = nullptr;
@@ -654,6 +655,19 @@ int check_resident(Engine &E) {
 
 // ------------------------------------------------------------ stage emitters
 
+// Whether the slice-interior column stage runs a wavefront per tile (col_wave)
+// instead of one per field (col_stage): from four wavefronts per CU on.  Per
+// launch, FP64: 62 instances of 2^13 16.0 -> 13.9 us, 64 of 2^14 23.2 -> 20.7
+// (4 samples per thread 27.1 -> 21.1), 61 of 2^15 36.2 -> 36.6 (44.1 -> 35.3),
+// two of 2^18 23.7 -> 17.7; below, the thinner launch loses: 62 of 2^12 (496
+// wavefronts) 13.2 -> 13.4, eight of 2^14 (256) 8.5 -> 10.7.  FP32C gains from
+// a few more on: 64 of 2^14 20.6 -> 16.1, 62 of 2^13 (992) 14.0 -> 13.9, 128 of
+// 2^12 (1024) 13.4 -> 13.6.
+bool wave_tiles(const Group &g) {
+  const long long waves = (long long)g.launch_n * g.N / (64 * g.ce);
+  return waves >= (g.fp32 ? 1100 : 960);
+}
+
 int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int store, int s_end, int s_start,
              int pump_off, int snap_every, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   RCHK(check_shapes(g));
@@ -666,6 +680,7 @@ int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int 
   a.xcd_pack = g.xcd_pack >= 0 ? g.xcd_pack : E.xcd_pack;
   a.swz = !a.xcd_pack && g.ct * esize(g) < 128 && (g.N2 / g.ct) % 8 == 0;
   a.spt = g.ce;
+  a.wave_tile = !E.solver && wave_tiles(g) && !(E.timing && g.fp32);
   if (engine_resident(E)) {  // the general kernel clears the next pass's counters (the slice-interior one ignores these)
     const Group &lead = res_follower(E, g) ? E.groups[0] : g;
     a.zero = reinterpret_cast<unsigned long long *>(lead.d_sync);
@@ -1505,9 +1520,10 @@ int engine_time_stages(Engine &E, Group &g, int iters, double *col_us, double *r
   return OPO_OK;
 }
 
-// FP32C is tuned on the two-launch path even where the pass runs resident: the
-// samples per thread and the phase source also decide how its results round,
-// and both paths then round alike.
+// FP32C is tuned on the two-launch path and its per-field column stage even
+// where the run takes the resident pass or wavefront tiles: the samples per
+// thread and the phase source also decide how its results round (1e-4 over
+// thousands of slices), and every path then rounds alike.
 bool time_resident(const Engine &E) { return engine_resident(E) && !E.fp32; }
 
 // n slices as a round trip of the group runs them, for timing: back-to-back
@@ -1524,11 +1540,14 @@ int time_some_slices(Engine &E, Group &g, int n) {
     return OPO_OK;
   }
   const int A = all_mask(g);
-  for (int it = 0; it < n; ++it) {
-    RCHK(emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, 0, 1 % E.NZ, 0, 0));
-    RCHK(emit_row(E, g, false, A));
+  int rc = OPO_OK;
+  E.timing = true;
+  for (int it = 0; it < n && rc == OPO_OK; ++it) {
+    rc = emit_col(E, g, OP_NL_END | OP_NL_START, A, A, A, A, 0, 1 % E.NZ, 0, 0);
+    if (rc == OPO_OK) rc = emit_row(E, g, false, A);
   }
-  return OPO_OK;
+  E.timing = false;
+  return rc;
 }
 
 // Average device time of one crystal slice as a round trip runs it: after a

@@ -69,18 +69,14 @@ template <typename V> __device__ __forceinline__ V mk(decltype(V::x) a, decltype
 }
 template <typename V> __device__ __forceinline__ V cadd(V a, V b) { return mk<V>(a.x + b.x, a.y + b.y); }
 template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>(a.x - b.x, a.y - b.y); }
-// Complex product.  FP64 by explicit fused multiply-adds: every kernel that
-// runs a stage (one launch per stage, or the resident pass) then rounds alike,
-// whatever the compiler would have contracted, and their results are the same
-// bit for bit.  (FP32 contracts alike in both as written; the tests compare.)
+// Complex product by explicit fused multiply-adds: every kernel that runs a
+// stage (a wavefront per field, a wavefront per tile, or the resident pass)
+// then rounds alike, whatever the compiler would have contracted, and their
+// results are the same bit for bit.
 __device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <typename V> __device__ __forceinline__ V cmul(V a, V b) {
-  if constexpr (std::is_same<V, double2>::value) {
-    return mk<V>(fma_(-a.y, b.y, a.x * b.x), fma_(a.x, b.y, a.y * b.x));
-  } else {
-    return mk<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-  }
+  return mk<V>(fma_(a.x, b.x, -(a.y * b.y)), fma_(a.y, b.x, a.x * b.y));
 }
 template <typename V> __device__ __forceinline__ V cconj(V a) { return mk<V>(a.x, -a.y); }
 template <typename V> __device__ __forceinline__ V cscale(V a, decltype(V::x) s) { return mk<V>(a.x * s, a.y * s); }
@@ -90,6 +86,13 @@ template <int S, typename V> __device__ __forceinline__ V mul_si(V a) {
 }
 // twiddle lookup from a table of e^{+2 pi i e/M}; conjugated for S < 0
 template <int S, typename V> __device__ __forceinline__ V tw_sign(V w) { return S > 0 ? w : cconj(w); }
+
+// u times the root w (conjugated for S < 0).  The operand order fixes which
+// product is rounded before the fused add; over thousands of slices FP32C
+// accumulates the difference to 1e-5, so it stays as it always was.
+template <int S, typename V> __device__ __forceinline__ V cmul_root(V u, V w) {
+  return S > 0 ? cmul(w, u) : cmul(u, cconj(w));
+}
 
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x >> 1); }
 // passes of radix E (E = 4 or 8 samples per thread), the last one of radix
@@ -224,7 +227,7 @@ __device__ __forceinline__ void fft_pass(V *v, bool on, V *buf0, int &ph, int t,
         } else {
 #pragma unroll
           for (int j = 1; j < R; ++j) {
-            if constexpr (TREG) u[j] = cmul(u[j], tw_sign<S>(tws[TOFF + b * (R - 1) + j - 1]));
+            if constexpr (TREG) u[j] = cmul_root<S>(u[j], tws[TOFF + b * (R - 1) + j - 1]);
             else u[j] = cmul(u[j], tw_sign<S>(tws[j * k * (M / (P * R))]));
           }
         }
@@ -340,9 +343,9 @@ __device__ __forceinline__ void nl_half_pt(V *xp, V *xs, V *xi, const NlCoef<NF,
 #pragma unroll
     for (int m = 0; m < K; ++m) {
       const V ap = xp[m], as = xs[m], ai = xi[m];
-      xp[m] = cadd(ap, cmul(Cp, cmul(as, ai)));
-      xs[m] = cadd(as, cmul(Cs, cmul(ap, cconj(ai))));
-      xi[m] = cadd(ai, cmul(Ci, cmul(ap, cconj(as))));
+      xp[m] = cadd(ap, cmul(cmul(as, ai), Cp));
+      xs[m] = cadd(as, cmul(cmul(ap, cconj(ai)), Cs));
+      xi[m] = cadd(ai, cmul(cmul(ap, cconj(as)), Ci));
     }
   } else {
     // cwes2.cuh:147-166: stages 2-4 evaluate dAdz on A + s*k (s = 0.5, 0.5, 1).

@@ -80,6 +80,7 @@ struct ColArgs {
   int xcd_pack;      // 1: grid is 8x wider and only blocks with blockIdx.x % 8 == 0 work
   int swz;           // 1: XCD-contiguous tile order (tiles narrower than a cache line)
   int spt;           // samples per thread of the column FFT (4 or 8)
+  int wave_tile;     // 1: slice interior with one wavefront per tile (col_wave)
   // counters of the resident pass that follows (opo_resident.h), cleared by
   // the general (boundary) kernel; null when none follows
   unsigned long long *zero;

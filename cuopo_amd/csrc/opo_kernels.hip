@@ -223,8 +223,8 @@ __global__ __launch_bounds__(E == 4 ? 1024 : 512) void col_stage(const OpoInst *
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const V e = eom[(long long)N2 * (t + (hb + q) * T1) + n2];
-          xs[q] = cmul(xs[q], e);
-          if constexpr (NF == 3) xi[q] = cmul(xi[q], e);
+          xs[q] = cmul(e, xs[q]);
+          if constexpr (NF == 3) xi[q] = cmul(e, xi[q]);
         }
       }
       if (ops & OP_MIRROR) {
@@ -233,8 +233,8 @@ __global__ __launch_bounds__(E == 4 ? 1024 : 512) void col_stage(const OpoInst *
         const R rs = (R)I->sqrt_rs, ri = (R)I->sqrt_ri;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          xs[q] = cmul(cscale(xs[q], rs), e);
-          if constexpr (NF == 3) xi[q] = cmul(cscale(xi[q], ri), e);
+          xs[q] = cmul(e, cscale(xs[q], rs));
+          if constexpr (NF == 3) xi[q] = cmul(e, cscale(xi[q], ri));
         }
       }
       if ((ops & OP_SAVE) || snap || (ops & OP_POWER)) {
@@ -326,6 +326,109 @@ __global__ __launch_bounds__(E == 4 ? 1024 : 512) void col_stage(const OpoInst *
   }
 }
 
+// One pass of the column transforms of all fields (see team_fft): while one
+// field's exchange is in flight the next field's butterflies run.
+template <int M, int S, int E, int NF, int Q = 0, typename V>
+__device__ __forceinline__ void wave_ffts(V (*v)[E], V *buf, int t, int c, int CT, const V *tw) {
+  if constexpr (Q < npasses(M, E)) {
+    int ph = 0;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) fft_pass<M, Q, S, false, false, E>(v[f], true, buf, ph, t, c, CT, 0, tw, true);
+    wave_ffts<M, S, E, NF, Q + 1>(v, buf, t, c, CT, tw);
+  }
+}
+
+// Slice-interior column stage, one wavefront per tile of 64*E/N1 columns with
+// every field in its registers.  Against col_stage<MID> (a wavefront per field,
+// fields meeting in LDS) a tile needs no meeting exchange and no block barrier,
+// forms the four-step twiddles once for all fields and moves 4.6 instead of 9.8
+// 16-byte values per sample through LDS; the arithmetic per field is the same,
+// and so are the bits.  222 VGPRs at 8 samples per thread in FP64 (2 wavefronts
+// per SIMD; three fields' worth of independent work in each), 118 at 4.  It has
+// a third of the wavefronts, so it pays where they still fill the chip
+// (wave_tiles in opo_api.cpp has the figures).
+template <typename T, int N1, int NF, int E>
+__global__ __launch_bounds__(256, 2) void col_wave(const OpoInst *__restrict__ insts, ColArgs a) {
+  using V = typename vec2<T>::type;
+  constexpr bool F64 = std::is_same<T, double>::value;
+  constexpr int T1 = N1 / E, CT = 64 / T1;
+  extern __shared__ unsigned char smem_raw[];
+  V *ltw = reinterpret_cast<V *>(smem_raw);  // N1-point root table, then 64*E values per wavefront
+  const OpoInst *I = insts + blockIdx.y;
+  if (I->active_v == 0) return;  // block-uniform
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+  V *buf = ltw + N1 + wave * 64 * E;
+  const int c = lane & (CT - 1), t = lane / CT;
+  const int N2 = a.N2;
+  const int n2 = ((int)blockIdx.x * waves + wave) * CT + c;
+  const long long N = (long long)N1 * N2;
+  const unsigned nmask = (unsigned)(N - 1);
+  const auto st = gp(reinterpret_cast<V *>(I->state)) + n2;
+  V v[NF][E];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[f][m] = st[f * N + (long long)N2 * (t + m * T1)];
+  const auto twlo = gp(reinterpret_cast<const V *>(a.twlo));
+  const auto twhi = gp(reinterpret_cast<const V *>(a.twhi));
+  const unsigned lm = (1u << a.lobits) - 1u;
+  V W[E], x0{}, b1{};
+  if constexpr (F64) {
+    const unsigned e0 = (unsigned)(n2 * t) & nmask, e1 = (unsigned)(n2 * T1) & nmask;
+    x0 = cmul(V(twhi[e0 >> a.lobits]), V(twlo[e0 & lm]));
+    b1 = cmul(V(twhi[e1 >> a.lobits]), V(twlo[e1 & lm]));
+  } else {
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const unsigned e = (unsigned)(n2 * (t + m * T1)) & nmask;
+      W[m] = cmul(V(twhi[e >> a.lobits]), V(twlo[e & lm]));
+    }
+  }
+  const NlCoef<NF, V> nle = load_nl<NF, V>(I->nl, I->h6, a.s_end), nls = load_nl<NF, V>(I->nl, I->h6, a.s_start);
+  {
+    const auto tw1 = gp(reinterpret_cast<const V *>(a.tw1));
+    for (int e = tid; e < N1; e += blockDim.x) ltw[e] = tw1[e];
+    __syncthreads();
+  }
+  // FP64: W_m = x0 b1^m as col_stage forms it, before either transform
+  auto roots = [&]() {
+    if constexpr (F64) {
+      const V b2 = cmul(b1, b1), b4 = cmul(b2, b2);
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        V w = x0;
+        if (m & 4) w = cmul(w, b4);
+        if (m & 2) w = cmul(w, b2);
+        if (m & 1) w = cmul(w, b1);
+        W[m] = w;
+      }
+    }
+  };
+  roots();
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[f][m] = cmul(v[f][m], cconj(W[m]));
+  wave_ffts<N1, -1, E, NF>(v, buf, t, c, CT, ltw);
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    V xi[1] = {NF == 3 ? v[NF - 1][m] : mk<V>(0, 0)};
+    nl_half_pt<NF, 1>(&v[0][m], &v[1][m], xi, nle);
+    nl_half_pt<NF, 1>(&v[0][m], &v[1][m], xi, nls);
+    if constexpr (NF == 3) v[2][m] = xi[0];
+  }
+  wave_ffts<N1, +1, E, NF>(v, buf, t, c, CT, ltw);
+  if constexpr (F64) {
+    asm volatile("" : "+v"(x0.x), "+v"(x0.y), "+v"(b1.x), "+v"(b1.y));  // form W again, as col_stage does
+    roots();
+  }
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int m = 0; m < E; ++m) st[f * N + (long long)N2 * (t + m * T1)] = cmul(v[f][m], W[m]);
+}
+
 // threads per row-stage block: a 4096-point row at 4 samples per thread needs 1024
 constexpr int row_max_threads(int N2, int E) { return (E == 4 && N2 >= 4096) ? 1024 : 512; }
 
@@ -374,9 +477,9 @@ __global__ __launch_bounds__(row_max_threads(N2, E)) void row_stage(const OpoIns
     const auto XH = S + N2;
     const auto XL = XH + ((N / E) >> L);
     const unsigned e = (unsigned)k1 * (unsigned)t;
-    xr = cmul(V(XH[e >> L]), V(XL[e & ((1u << L) - 1u)]));
+    xr = cmul(V(XL[e & ((1u << L) - 1u)]), V(XH[e >> L]));
 #pragma unroll
-    for (int m = 0; m < E; ++m) ph_tab[m] = cmul(V(F[E * k1 + m]), V(S[t + m * T2]));
+    for (int m = 0; m < E; ++m) ph_tab[m] = cmul(V(S[t + m * T2]), V(F[E * k1 + m]));
   } else {
     tab = tab + (long long)N2 * k1;
 #pragma unroll
@@ -387,7 +490,7 @@ __global__ __launch_bounds__(row_max_threads(N2, E)) void row_stage(const OpoIns
   load_twiddles<N2, E>(treg, t, gp(reinterpret_cast<const V *>(a.tw2)));
   if (use_fac) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) ph_tab[m] = cmul(ph_tab[m], xr);
+    for (int m = 0; m < E; ++m) ph_tab[m] = cmul(xr, ph_tab[m]);
   }
   int ph = 0;
   const int bufstride = RT * NP2;
@@ -481,6 +584,16 @@ static int launch_col_e(int ct, int count, const OpoInst *insts, const ColArgs &
   using V = typename vec2<T>::type;
   dim3 grid((a.N2 / ct) * (a.xcd_pack ? 8 : 1), count);
   const bool mid = col_is_mid<NF>(a);
+  if (mid && a.wave_tile) {
+    constexpr int CT = 64 * E / N1;
+    const int tiles = a.N2 / CT, waves = tiles < 4 ? tiles : 4;
+    if (a.N2 % CT != 0 || tiles % waves != 0) return (int)hipErrorInvalidValue;
+    const size_t bytes = ((size_t)N1 + (size_t)waves * 64 * E) * sizeof(V);
+    auto k = &col_wave<T, N1, NF, E>;
+    if (e0 || e1) hipExtLaunchKernelGGL(k, dim3(tiles / waves, count), dim3(64 * waves), bytes, s, e0, e1, 0, insts, a);
+    else hipLaunchKernelGGL(k, dim3(tiles / waves, count), dim3(64 * waves), bytes, s, insts, a);
+    return (int)hipGetLastError();
+  }
   // one exchange buffer when the slice-interior kernel's field teams are
   // single wavefronts (the rule col_stage applies), two otherwise
   const int nbuf = (mid && team_in_wave(ct * (N1 / E))) ? 1 : 2;

@@ -243,9 +243,9 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
             const auto XH = Sx + N2;
             const auto XL = XH + ((N / ER) >> L);
             const unsigned e = (unsigned)k1 * (unsigned)t;
-            xr = cmul(V(XH[e >> L]), V(XL[e & ((1u << L) - 1u)]));
+            xr = cmul(V(XL[e & ((1u << L) - 1u)]), V(XH[e >> L]));
 #pragma unroll
-            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(V(F[ER * k1 + m]), V(Sx[t + m * T2]));
+            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(V(Sx[t + m * T2]), V(F[ER * k1 + m]));
           } else {
 #pragma unroll
             for (int m = 0; m < ER; ++m) ph_tab[m] = lin[row + t + m * T2];
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
           for (int m = 0; m < ER; ++m) v[m] = in.load(row + t + m * T2);
           if (use_fac) {
 #pragma unroll
-            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(ph_tab[m], xr);
+            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(xr, ph_tab[m]);
           }
           int ph = 0;
           constexpr int NP2 = N2 + N2 / 8;

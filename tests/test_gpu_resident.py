@@ -120,3 +120,40 @@ def test_resident_solvers_side_by_side(gpu):
     for k in range(len(cfgs)):
         assert all(np.array_equal(a, b) for a, b in zip(alone[k], beside[k])), k
         assert rel_l2(alone[k][1], beside[k][1]) == 0
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("config", [c1, c2])
+@pytest.mark.parametrize("N,count,ce", [(512, 1100, 8), (1024, 600, 8), (4096, 140, 8), (4096, 70, 4), (32768, 18, 8),
+                                        (65536, 9, 8), (262144, 2, 8), (262144, 2, 4)])
+def test_wavefront_tiles_give_the_same_bits(gpu, monkeypatch, N, count, ce, config, fp32):
+    """Batches whose column stage runs a wavefront per tile (every column length, 8 and 4 samples per thread)
+    against the same instances alone, whose launches are below that rule and run one per field."""
+    P = gpu
+    monkeypatch.setenv("OPO_RESIDENT", "0")  # both launch stage by stage
+    monkeypatch.setenv("OPO_SPLIT", "0")  # and the batch as one group
+    prec = P.FP32C if fp32 else P.FP64
+    cfgs = []
+    for k in range(5):
+        c = config(N=N, NZ=3, NRT=3)
+        c.Nth = 1.5 + 0.5 * k
+        cfgs.append(c)
+    made = []
+    for k, c in enumerate(cfgs):
+        p, T, w, Ap_in, Ap, As, Ai = inputs(c, seed=80 + k, sigma=1e-3)
+        made.append((P.params_from(P.derive(to_args(c)), prec), w, T, Ap_in, Ap, As, Ai))
+
+    def run(n):
+        b = P.Batch([made[k % len(made)][0] for k in range(n)])
+        for k in range(n):
+            b.upload(k, *made[k % len(made)][1:])
+        b.set_tuning(N, col_spt=ce, phase_mode=0)
+        b.run(2, check_every=0, tol=0.0)
+        out = [b.download(k) for k in ({0, 1, n - 1} if n > 1 else {0})]
+        b.close()
+        return out
+
+    many, one = run(count), run(1)
+    for f, g in zip(many[0], one[0]):
+        assert (f is None and g is None) or np.array_equal(f, g)
+    assert all(np.isfinite(f).all() for x in many for f in x if f is not None)
