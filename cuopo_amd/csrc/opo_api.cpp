@@ -296,6 +296,17 @@ int check_shapes(const Group &g) {
   return OPO_OK;
 }
 
+// Counters of the one-launch crystal passes.  In the no-allocation mode they
+// take what the scratch has left; without them the pass runs stage by stage.
+int alloc_sync(Engine &E, Group &g) {
+  if (!E.resident || !opo::resident_supported(g.N1, g.N2, 8, 8)) return OPO_OK;
+  if (g.pool && g.pool_cap - g.pool_used < sizeof(opo::ResSync) + 1024) return OPO_OK;
+  RCHK(dalloc(g, (void **)&g.d_sync, sizeof(opo::ResSync)));
+  RCHK(dalloc(g, (void **)&g.d_err, 8));
+  const int e = opo::launch_zero(g.d_err, 1, E.stream);
+  return e == 0 ? OPO_OK : fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
+}
+
 int make_group(Engine &E, Group &g) {
   g.NF = E.three_eqs ? 3 : 2;
   g.fp32 = E.fp32;
@@ -338,12 +349,7 @@ int make_group(Engine &E, Group &g) {
   } else {
     HIPCHK(hipMemsetAsync(g.d_hist, 0, (size_t)n * g.hist_len * sizeof(double), E.stream));
   }
-  if (E.resident && opo::resident_supported(g.N1, g.N2, 8, 8)) {
-    RCHK(dalloc(g, (void **)&g.d_sync, sizeof(opo::ResSync)));
-    RCHK(dalloc(g, (void **)&g.d_err, 8));
-    const int e = opo::launch_zero(g.d_err, 1, E.stream);
-    if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
-  }
+  if (!g.pool) RCHK(alloc_sync(E, g));
   g.inst.resize(n);
   for (int k = 0; k < n; ++k) {
     Instance &I = g.inst[k];
@@ -1444,6 +1450,8 @@ int opo_run_noalloc(const opo_params *params, const double *w, const double *T, 
   RCHK(make_group(E, g));
   g.inst[0].prm = *params;
   RCHK(upload_instance(E, g, 0, w, T, nullptr, n_ap, nullptr, nullptr, nullptr));
+  if (const char *rs = std::getenv("OPO_RESIDENT")) E.resident = rs[0] != '0';
+  RCHK(alloc_sync(E, g));  // last: it never takes what the instance needs
   RCHK(engine_run(E, rt0, n_rt, 0, 0.0));
   if (power_out) {
     HIPCHK(hipMemcpyAsync(power_out, g.d_hist + rt0, (size_t)n_rt * sizeof(double), hipMemcpyDeviceToHost,

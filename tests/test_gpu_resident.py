@@ -157,3 +157,42 @@ def test_wavefront_tiles_give_the_same_bits(gpu, monkeypatch, N, count, ce, conf
     for f, g in zip(many[0], one[0]):
         assert (f is None and g is None) or np.array_equal(f, g)
     assert all(np.isfinite(f).all() for x in many for f in x if f is not None)
+
+
+def test_noalloc_scratch_holds_as_much_as_without_the_counters(gpu, monkeypatch):
+    """The one-launch pass takes its counters from what the scratch has left: the longest power history that the
+    scratch holds is the same with and without it, and so are the results just above and below."""
+    import ctypes as C
+
+    from tests.test_zz_no_alloc import Dev, hip
+
+    P = gpu
+    cfg = c1(N=1024, NZ=3, NRT=4)
+    p, T, w, Ap_in, Ap, As, _ = inputs(cfg, seed=9, sigma=1e-3)
+    prm = P.params_from(P.derive(to_args(cfg)))
+    h = hip()
+
+    def run(rt0):
+        df, dp = Dev(h, np.concatenate([Ap, As])), Dev(h, np.ascontiguousarray(Ap_in))
+        try:
+            rc = P.lib().opo_run_noalloc(C.byref(prm), w.ctypes.data_as(C.c_void_p), T.ctypes.data_as(C.c_void_p),
+                                         dp.p, Ap_in.size, df.p, rt0, 1, None, None)
+            return df.get(2 * cfg.N) if rc == P.OK else None
+        finally:
+            df.free()
+            dp.free()
+
+    def longest():
+        lo, hi = 0, 1 << 21  # 16 MiB of history: more than the scratch
+        assert run(hi) is None
+        while hi - lo > 1:
+            mid = (lo + hi) // 2
+            lo, hi = (mid, hi) if run(mid) is not None else (lo, mid)
+        return lo
+
+    monkeypatch.setenv("OPO_RESIDENT", "0")
+    want, field = longest(), run(0)
+    monkeypatch.setenv("OPO_RESIDENT", "1")
+    assert longest() == want
+    for rt0 in (0, want - (1 << 15), want - 64, want):
+        assert np.array_equal(run(rt0), field)
