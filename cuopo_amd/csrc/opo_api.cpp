@@ -299,7 +299,8 @@ int check_shapes(const Group &g) {
 // Counters of the one-launch crystal passes.  In the no-allocation mode they
 // take what the scratch has left; without them the pass runs stage by stage.
 int alloc_sync(Engine &E, Group &g) {
-  if (!E.resident || !opo::resident_supported(g.N1, g.N2, 8, 8)) return OPO_OK;
+  if (!E.resident || !(opo::resident_supported(g.N1, g.N2, 8, 8) || opo::chip_supported(g.N1, g.N2, 8, 8, g.fp32)))
+    return OPO_OK;
   if (g.pool && g.pool_cap - g.pool_used < sizeof(opo::ResSync) + 1024) return OPO_OK;
   RCHK(dalloc(g, (void **)&g.d_sync, sizeof(opo::ResSync)));
   RCHK(dalloc(g, (void **)&g.d_err, 8));
@@ -594,9 +595,19 @@ ResShape res_shape(const Engine &E, const Group &g) { return res_shape(g, res_co
 constexpr long long kResTurn = 1LL << 19;  // samples of one turn of every XCD's teams
 constexpr double kResTurnUs = 16.5, kStreamUs = 7.0, kStreamUsPerSample = 31e-6;
 
+// One instance of 2^15 samples or more with 8 samples per thread: the whole
+// chip works on it (opo_chip.h: 1.2 to 1.4 times the two-launch path, 1.1
+// times one XCD's team at 2^15).  Below, rows no longer fill a wavefront and
+// one XCD's barrier is the cheaper one (2^14: 7.0 us a slice); several
+// instances fill the chip stage by stage.
+bool chip_wide(const Engine &E, const Group &g) {
+  return E.groups.size() == 1 && g.launch_n == 1 && opo::chip_supported(g.N1, g.N2, g.ce, g.re, g.fp32);
+}
+
 bool engine_resident(const Engine &E) {
   if (!E.resident || E.groups.empty()) return false;
   const Group &g = E.groups[0];
+  if (g.d_sync && chip_wide(E, g)) return true;
   if (!g.d_sync || (E.groups.size() != 1 && !res_second(E, g))) return false;
   for (const auto &h : E.groups)
     if (!opo::resident_supported(h.N1, h.N2, h.ce, h.re)) return false;
@@ -609,9 +620,9 @@ bool engine_resident(const Engine &E) {
   return (count + turn - 1) / turn * kResTurnUs < kStreamUs + kStreamUsPerSample * (double)samples;
 }
 
-// 8-byte words of the counters that a pass of this shape uses
-int res_sync_words(const ResShape &r) {
-  return (int)((offsetof(opo::ResSync, team) + sizeof(opo::ResTeam) * (size_t)(r.teams * opo::kXcds)) / 8);
+// 8-byte words of the counters that a pass with this many team lines uses
+int res_sync_words(int lines) {
+  return (int)((offsetof(opo::ResSync, team) + sizeof(opo::ResTeam) * (size_t)lines) / 8);
 }
 
 int clear_sync(Group &g, hipStream_t st) {
@@ -638,6 +649,11 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   a.prefer = (int)((reinterpret_cast<uintptr_t>(g.d_insts) >> 12) % opo::kXcds);
   a.sync = g.d_sync;
   a.err = g.d_err;
+  if (chip_wide(E, g)) {
+    const int e = opo::launch_chip(g.fp32, g.N1, g.N2, g.NF, g.d_insts, a, g.cur);
+    if (e != 0) return fail(OPO_ERR_HIP, std::string("chip pass launch: ") + hipGetErrorString((hipError_t)e));
+    return OPO_OK;
+  }
   const int e = opo::launch_resident(g.fp32, g.N1, g.N2, g.NF, r.ce, r.re, g.d_insts, a, r.blocks * opo::kXcds, g.cur);
   if (e != 0) return fail(OPO_ERR_HIP, std::string("resident pass launch: ") + hipGetErrorString((hipError_t)e));
   return OPO_OK;
@@ -690,7 +706,7 @@ int emit_col(Engine &E, Group &g, unsigned ops, int load, int inv, int fwd, int 
   if (engine_resident(E)) {  // the general kernel clears the next pass's counters (the slice-interior one ignores these)
     const Group &lead = res_follower(E, g) ? E.groups[0] : g;
     a.zero = reinterpret_cast<unsigned long long *>(lead.d_sync);
-    a.zero_words = res_sync_words(res_shape(E, lead));
+    a.zero_words = chip_wide(E, lead) ? res_sync_words(opo::kChipCounters) : res_sync_words(res_shape(E, lead).teams * opo::kXcds);
   }
   if (E.solver) {
     const Instance &I = g.inst[0];

@@ -112,8 +112,10 @@ constexpr int kXcds = 8, kMaxTeams = 32;  // teams per XCD
 struct alignas(128) ResLine {
   unsigned v;
 };
+struct alignas(128) ResLine128 { unsigned v; };
+constexpr int kTeamCounters = 1;
 struct ResTeam {
-  alignas(128) unsigned done;            // stages finished, summed over the team's blocks
+  ResLine128 part[kTeamCounters];        // stages finished, summed over the team's blocks (block b: part b mod kTeamCounters)
   alignas(128) unsigned long long cur;   // (turn << 32) | instance the team works on
 };
 struct ResSync {
@@ -138,6 +140,10 @@ struct ResArgs {
 // threads per block of the resident pass
 constexpr int res_max_threads(int, int) { return 768; }
 bool resident_supported(int N1, int N2, int ce, int re);
+constexpr int kChipBlocks = 256;  // one per CU
+constexpr int kChipCounters = 64;
+bool chip_supported(int N1, int N2, int ce, int re, int fp32);
+int launch_chip(int fp32, int N1, int N2, int NF, const OpoInst *insts, const ResArgs &a, void *stream);
 int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoInst *insts, const ResArgs &a, int grid,
                     void *stream);
 

@@ -68,8 +68,9 @@ template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *
 // scope.  `off` in elements.
 template <typename V> struct FieldBuf {
   __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ FieldBuf(void *base, unsigned bytes)
-      : r(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00020000)) {}
+  V *base;
+  __device__ __forceinline__ FieldBuf(V *p, unsigned bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000)), base(p) {}
   __device__ __forceinline__ V load(unsigned off) const {
     constexpr int kAgent = 16;  // sc1
     if constexpr (sizeof(V) == 16) {
@@ -80,6 +81,18 @@ template <typename V> struct FieldBuf {
       typedef unsigned u2 __attribute__((ext_vector_type(2)));
       const u2 w = __builtin_amdgcn_raw_buffer_load_b64(r, (int)(off * 8), 0, kAgent);
       return __builtin_bit_cast(V, w);
+    }
+  }
+  // WIDE: past this XCD's L2 as well (agent scope), for readers on the others
+  template <bool WIDE> __device__ __forceinline__ void store(unsigned off, V v) const {
+    if constexpr (!WIDE) {
+      gp(base)[off] = v;
+    } else if constexpr (sizeof(V) == 16) {
+      typedef unsigned u4 __attribute__((ext_vector_type(4)));
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, (int)(off * 16), 0, 16);
+    } else {
+      typedef unsigned u2 __attribute__((ext_vector_type(2)));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)(off * 8), 0, 16);
     }
   }
 };
@@ -98,16 +111,160 @@ template <int NF, int EC, int ER> __host__ __device__ constexpr int res_tile_ele
   return NF * (64 * EC > 72 * ER ? 64 * EC : 72 * ER);  // rows carry one pad slot per 8 samples
 }
 
+// Row k1 of field f by the thread's team of N2/ER threads (t: its index):
+// FFT, linear phase, inverse FFT.  `on`: there is such a row; `mine`: the
+// thread has a part of the LDS.  `wait` returns once the stage before is
+// complete; phases and twiddles are constant, so their loads go out before.
+template <int N1, int N2, int ER, bool WIDE, typename V, typename D, typename Wait>
+__device__ __forceinline__ bool row_tile(const FieldBuf<V> &in, const ResArgs &a, D I, int f, int k1, int t, bool on,
+                                         bool mine, V *buf, int gbase, int bufstride, Wait wait) {
+  constexpr unsigned N = N1 * N2;
+  constexpr int T2 = N2 / ER;
+  constexpr bool wave = team_in_wave(T2);
+  const unsigned row = f * N + N2 * k1;
+  constexpr int NTW = tw_count(N2, ER, tw_pow<V>());
+  V v[ER], ph_tab[ER], treg[NTW > 0 ? NTW : 1];
+  V xr = mk<V>(0, 0);
+  const auto lfac = gp(reinterpret_cast<const V *>(I->lfac_spt[ER == 8 ? 0 : 1]));
+  const bool use_fac = (bool)lfac;
+  if (use_fac) {
+    const int L = a.xl_bits;
+    const long long FB = (long long)ER * N1 + N2 + ((N / ER) >> L) + (1LL << L);
+    const auto F = lfac + f * FB;
+    const auto Sx = F + ER * N1;
+    const auto XH = Sx + N2;
+    const auto XL = XH + ((N / ER) >> L);
+    const unsigned e = (unsigned)k1 * (unsigned)t;
+    xr = cmul(V(XL[e & ((1u << L) - 1u)]), V(XH[e >> L]));
+#pragma unroll
+    for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(V(Sx[t + m * T2]), V(F[ER * k1 + m]));
+  } else {
+    const auto lin = gp(reinterpret_cast<const V *>(I->lin));
+#pragma unroll
+    for (int m = 0; m < ER; ++m) ph_tab[m] = lin[row + t + m * T2];
+  }
+  load_twiddles<N2, ER>(treg, t, gp(reinterpret_cast<const V *>(a.tw2)));
+  if (!wait()) return false;
+#pragma unroll
+  for (int m = 0; m < ER; ++m) v[m] = in.load(row + t + m * T2);
+  if (use_fac) {
+#pragma unroll
+    for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(xr, ph_tab[m]);
+  }
+  int ph = 0;
+  team_fft<N2, +1, true, true, ER>(v, mine, buf, ph, t, gbase, 1, bufstride, treg, wave);
+#pragma unroll
+  for (int m = 0; m < ER; ++m) v[m] = cmul(v[m], ph_tab[m]);
+  team_fft<N2, -1, true, true, ER>(v, mine, buf, ph, t, gbase, 1, bufstride, treg, wave);
+  if (on) {
+#pragma unroll
+    for (int m = 0; m < ER; ++m) in.template store<WIDE>(row + t + m * T2, v[m]);
+  }
+  return true;
+}
+
+// Field f of one tile of 64*EC/N1 columns, one wavefront: inverse FFT, NL end
+// of slice s, NL start of s + 1 (over the tile's NF wavefronts), FFT.
+template <int N1, int N2, int NF, int EC, bool WIDE, typename V, typename Wait>
+__device__ __forceinline__ bool col_tile(const FieldBuf<V> &in, const ResArgs &a, int f, int tile, int lane, bool on,
+                                         bool mine, V *lds, const V *ltw, const NlCoef<NF, V> &nle,
+                                         const NlCoef<NF, V> &nls, Wait wait) {
+  constexpr bool F64 = sizeof(V) == 16;
+  constexpr unsigned N = N1 * N2;
+  constexpr int T1 = N1 / EC, CT = 64 / T1;
+  constexpr int fstride = 64 * EC;
+  const int c = lane & (CT - 1), t = lane / CT;
+  const int n2 = (on ? tile : 0) * CT + c;
+  const unsigned at = f * N + n2;
+  const auto twlo = gp(reinterpret_cast<const V *>(a.twlo));
+  const auto twhi = gp(reinterpret_cast<const V *>(a.twhi));
+  const unsigned lm = (1u << a.lobits) - 1u;
+  // four-step twiddles as col_stage forms them (same products)
+  V gh[F64 ? 1 : EC], gl[F64 ? 1 : EC], W[EC];
+  V x0{}, b1{};
+  if constexpr (F64) {
+    const unsigned e0 = (unsigned)(n2 * t) & (N - 1), e1 = (unsigned)(n2 * T1) & (N - 1);
+    const V x0h = twhi[e0 >> a.lobits], x0l = twlo[e0 & lm];
+    const V b1h = twhi[e1 >> a.lobits], b1l = twlo[e1 & lm];
+    x0 = cmul(x0h, x0l);
+    b1 = cmul(b1h, b1l);
+  } else {
+#pragma unroll
+    for (int m = 0; m < EC; ++m) {
+      const unsigned e = (unsigned)(n2 * (t + m * T1)) & (N - 1);
+      gh[m] = twhi[e >> a.lobits];
+      gl[m] = twlo[e & lm];
+    }
+#pragma unroll
+    for (int m = 0; m < EC; ++m) W[m] = cmul(gh[m], gl[m]);
+  }
+  if (!wait()) return false;
+  V v[EC];
+#pragma unroll
+  for (int m = 0; m < EC; ++m) v[m] = in.load(at + N2 * (t + m * T1));
+  auto roots = [&]() {
+    if constexpr (F64) {
+      const V b2 = cmul(b1, b1), b4 = cmul(b2, b2);
+#pragma unroll
+      for (int m = 0; m < EC; ++m) {
+        V w = x0;
+        if (m & 4) w = cmul(w, b4);
+        if (m & 2) w = cmul(w, b2);
+        if (m & 1) w = cmul(w, b1);
+        W[m] = w;
+      }
+    }
+  };
+  roots();
+  int ph = 0;
+  V *own = lds + f * fstride;
+#pragma unroll
+  for (int m = 0; m < EC; ++m) v[m] = cmul(v[m], cconj(W[m]));
+  team_fft<N1, -1, false, false, EC>(v, mine, own, ph, t, c, CT, 0, ltw, true);
+#pragma unroll
+  for (int m = 0; m < EC; ++m)
+    if (mine) own[c + (t + m * T1) * CT] = v[m];
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < EC; ++m) {
+    if (mine && m % NF == f) {
+      const int o = c + (t + m * T1) * CT;
+      V xp[1] = {lds[o]}, xq[1] = {lds[fstride + o]};
+      V xi[1] = {NF == 3 ? lds[2 * fstride + o] : mk<V>(0, 0)};
+      nl_half_pt<NF, 1>(xp, xq, xi, nle);
+      nl_half_pt<NF, 1>(xp, xq, xi, nls);
+      lds[o] = xp[0];
+      lds[fstride + o] = xq[0];
+      if constexpr (NF == 3) lds[2 * fstride + o] = xi[0];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < EC; ++m) v[m] = own[c + (t + m * T1) * CT];
+  team_fft<N1, +1, false, false, EC>(v, mine, own, ph, t, c, CT, 0, ltw, true);
+  if constexpr (F64) {
+    // W again from its two roots (see col_stage)
+    asm volatile("" : "+v"(x0.x), "+v"(x0.y), "+v"(b1.x), "+v"(b1.y));
+    roots();
+  }
+#pragma unroll
+  for (int m = 0; m < EC; ++m) v[m] = cmul(v[m], W[m]);
+  if (on) {
+#pragma unroll
+    for (int m = 0; m < EC; ++m) in.template store<WIDE>(at + N2 * (t + m * T1), v[m]);
+  }
+  return true;
+}
+
 template <typename T, int N1, int N2, int NF, int EC, int ER>
 __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const OpoInst *__restrict__ insts, ResArgs a) {
   using V = typename vec2<T>::type;
-  constexpr bool F64 = std::is_same<T, double>::value;
   constexpr int T1 = N1 / EC, T2 = N2 / ER;
   constexpr int CT = 64 / T1, RT = 64 / T2;
   constexpr int NTC = N2 / CT, NTR = N1 / RT;
   constexpr unsigned N = N1 * N2;
   static_assert(T1 <= 64 && T2 <= 64 && NTC >= 1 && NTR >= 1, "one wavefront per field");
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];  // (the static words before it are not a multiple of 16 bytes)
   __shared__ unsigned long long sh_next[2];
   __shared__ int sh_rank, sh_size, sh_ok;
   V *ltw = reinterpret_cast<V *>(smem_raw);  // N1-point root table
@@ -158,7 +315,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
   const int size = min(per, xs - team * per);
   ResTeam *tm = &S->team[team * kXcds + x];
   const int nsub = a.sub, workers = size * nsub;
-  unsigned arrived = 0;  // barrier target: arrivals of this team so far
+  unsigned arrived = 0;  // stages finished
 
   for (unsigned epoch = 1;; ++epoch) {
     // ---- the team's next instance ----
@@ -188,10 +345,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
     const auto I = cp_scalar(idx < (unsigned)a.count ? insts + idx : a.insts2 + (idx - (unsigned)a.count));
     if (I->active_v == 0) continue;
     V *state = reinterpret_cast<V *>(I->state);
-    const auto st = gp(state);
     const FieldBuf<V> in(state, NF * N * (unsigned)sizeof(V));
-    const auto lfac = gp(reinterpret_cast<const V *>(I->lfac_spt[ER == 8 ? 0 : 1]));
-    const auto lin = gp(reinterpret_cast<const V *>(I->lin));
     const double *nl = I->nl;
     const double h6 = I->h6;
     bool first = true;
@@ -202,11 +356,19 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
         first = false;
         return true;
       }
-      if (tid == 0) {
-        const unsigned need = arrived;
-        const bool ok = poll_until(&tm->done, [need](unsigned v) { return (int)(v - need) >= 0; });
-        if (!ok) agent_store(&a.err[0], 3);
-        sh_ok = ok;
+      if (tid < 64) {
+        const int c = lane & (kTeamCounters - 1);
+        const unsigned need = arrived * (unsigned)((size + kTeamCounters - 1 - c) / kTeamCounters);
+        bool ok = false;
+        for (unsigned n = 0; n < kMaxPolls && !ok; ++n) {
+          ok = lane >= kTeamCounters || (int)(agent_load(&tm->part[c].v) - need) >= 0;
+          ok = __all(ok);
+          if (!ok) __builtin_amdgcn_s_sleep(1);
+        }
+        if (tid == 0) {
+          if (!ok) agent_store(&a.err[0], 3);
+          sh_ok = ok;
+        }
       }
       __syncthreads();
       return __builtin_amdgcn_readfirstlane(sh_ok) != 0;
@@ -215,8 +377,8 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
     auto arrive = [&]() {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (tid == 0) agent_add(&tm->done, 1u);
-      arrived += (unsigned)size;
+      if (tid == 0) agent_add(&tm->part[r0 & (kTeamCounters - 1)].v, 1u);
+      ++arrived;
     };
 
     for (int s = 0; s < a.NZ; ++s) {
@@ -225,152 +387,32 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
         const int l = opaque(lane);
         const int t = l & (T2 - 1), r = l / T2;
         bool waited = false;
+        auto wait = [&]() { return waited || (waited = wait_team()); };
         for (int t0 = 0; t0 < NTR; t0 += workers) {
           const int tile = t0 + r0 * nsub + sub;
           const bool on = tile < NTR;
           const int k1 = (on ? tile : 0) * RT + r;
-          const unsigned row = f * N + N2 * k1;
-          constexpr int NTW = tw_count(N2, ER, tw_pow<V>());
-          V v[ER], ph_tab[ER], treg[NTW > 0 ? NTW : 1];
-          V xr = mk<V>(0, 0);
-          const bool use_fac = (bool)lfac;
-          // phases and twiddles are constant: their loads go out before the wait
-          if (use_fac) {
-            const int L = a.xl_bits;
-            const long long FB = (long long)ER * N1 + N2 + ((N / ER) >> L) + (1LL << L);
-            const auto F = lfac + f * FB;
-            const auto Sx = F + ER * N1;
-            const auto XH = Sx + N2;
-            const auto XL = XH + ((N / ER) >> L);
-            const unsigned e = (unsigned)k1 * (unsigned)t;
-            xr = cmul(V(XL[e & ((1u << L) - 1u)]), V(XH[e >> L]));
-#pragma unroll
-            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(V(Sx[t + m * T2]), V(F[ER * k1 + m]));
-          } else {
-#pragma unroll
-            for (int m = 0; m < ER; ++m) ph_tab[m] = lin[row + t + m * T2];
-          }
-          load_twiddles<N2, ER>(treg, t, gp(reinterpret_cast<const V *>(a.tw2)));
-          if (!waited) {
-            if (!wait_team()) return;
-            waited = true;
-          }
-#pragma unroll
-          for (int m = 0; m < ER; ++m) v[m] = in.load(row + t + m * T2);
-          if (use_fac) {
-#pragma unroll
-            for (int m = 0; m < ER; ++m) ph_tab[m] = cmul(xr, ph_tab[m]);
-          }
-          int ph = 0;
-          constexpr int NP2 = N2 + N2 / 8;
           V *buf = lds + f * (64 * ER + 8 * ER);
-          team_fft<N2, +1, true, true, ER>(v, true, buf, ph, t, r * NP2, 1, 0, treg, true);
-#pragma unroll
-          for (int m = 0; m < ER; ++m) v[m] = cmul(v[m], ph_tab[m]);
-          team_fft<N2, -1, true, true, ER>(v, true, buf, ph, t, r * NP2, 1, 0, treg, true);
-          if (on) {
-#pragma unroll
-            for (int m = 0; m < ER; ++m) st[row + t + m * T2] = v[m];
-          }
+          constexpr int NP2 = N2 + N2 / 8;
+          if (!row_tile<N1, N2, ER, false>(in, a, I, f, k1, t, on, true, buf, r * NP2, 0, wait)) return;
         }
-        if (!waited && !wait_team()) return;  // (a block without a tile still keeps step)
+        if (!wait()) return;  // (a block without a tile still keeps step)
         arrive();
       }
       if (s == a.NZ - 1) break;
       // ---- column stage: inverse FFT, NL end of slice s, NL start of s + 1, FFT ----
       {
         const int l = opaque(lane);
-        const int c = l & (CT - 1), t = l / CT;
         const NlCoef<NF, V> nle = load_nl_at<NF, V>(cp_scalar(nl) + 16 * s, h6);
         const NlCoef<NF, V> nls = load_nl_at<NF, V>(cp_scalar(nl) + 16 * (s + 1), h6);
-        constexpr int fstride = 64 * EC;
         bool waited = false;
+        auto wait = [&]() { return waited || (waited = wait_team()); };
         for (int t0 = 0; t0 < NTC; t0 += workers) {
           const int tile = t0 + r0 * nsub + sub;
           const bool on = tile < NTC;
-          const int n2 = (on ? tile : 0) * CT + c;
-          const unsigned at = f * N + n2;
-          const auto twlo = gp(reinterpret_cast<const V *>(a.twlo));
-          const auto twhi = gp(reinterpret_cast<const V *>(a.twhi));
-          const unsigned lm = (1u << a.lobits) - 1u;
-          // four-step twiddles as col_stage forms them (same products)
-          V gh[F64 ? 1 : EC], gl[F64 ? 1 : EC], W[EC];
-          V x0{}, b1{};
-          if constexpr (F64) {
-            const unsigned e0 = (unsigned)(n2 * t) & (N - 1), e1 = (unsigned)(n2 * T1) & (N - 1);
-            const V x0h = twhi[e0 >> a.lobits], x0l = twlo[e0 & lm];
-            const V b1h = twhi[e1 >> a.lobits], b1l = twlo[e1 & lm];
-            x0 = cmul(x0h, x0l);
-            b1 = cmul(b1h, b1l);
-          } else {
-#pragma unroll
-            for (int m = 0; m < EC; ++m) {
-              const unsigned e = (unsigned)(n2 * (t + m * T1)) & (N - 1);
-              gh[m] = twhi[e >> a.lobits];
-              gl[m] = twlo[e & lm];
-            }
-#pragma unroll
-            for (int m = 0; m < EC; ++m) W[m] = cmul(gh[m], gl[m]);
-          }
-          if (!waited) {
-            if (!wait_team()) return;
-            waited = true;
-          }
-          V v[EC];
-#pragma unroll
-          for (int m = 0; m < EC; ++m) v[m] = in.load(at + N2 * (t + m * T1));
-          auto roots = [&]() {
-            if constexpr (F64) {
-              const V b2 = cmul(b1, b1), b4 = cmul(b2, b2);
-#pragma unroll
-              for (int m = 0; m < EC; ++m) {
-                V w = x0;
-                if (m & 4) w = cmul(w, b4);
-                if (m & 2) w = cmul(w, b2);
-                if (m & 1) w = cmul(w, b1);
-                W[m] = w;
-              }
-            }
-          };
-          roots();
-          int ph = 0;
-          V *mine = lds + f * fstride;
-#pragma unroll
-          for (int m = 0; m < EC; ++m) v[m] = cmul(v[m], cconj(W[m]));
-          team_fft<N1, -1, false, false, EC>(v, true, mine, ph, t, c, CT, 0, ltw, true);
-#pragma unroll
-          for (int m = 0; m < EC; ++m) mine[c + (t + m * T1) * CT] = v[m];
-          __syncthreads();
-#pragma unroll
-          for (int m = 0; m < EC; ++m) {
-            if (m % NF == f) {
-              const int o = c + (t + m * T1) * CT;
-              V xp[1] = {lds[o]}, xq[1] = {lds[fstride + o]};
-              V xi[1] = {NF == 3 ? lds[2 * fstride + o] : mk<V>(0, 0)};
-              nl_half_pt<NF, 1>(xp, xq, xi, nle);
-              nl_half_pt<NF, 1>(xp, xq, xi, nls);
-              lds[o] = xp[0];
-              lds[fstride + o] = xq[0];
-              if constexpr (NF == 3) lds[2 * fstride + o] = xi[0];
-            }
-          }
-          __syncthreads();
-#pragma unroll
-          for (int m = 0; m < EC; ++m) v[m] = mine[c + (t + m * T1) * CT];
-          team_fft<N1, +1, false, false, EC>(v, true, mine, ph, t, c, CT, 0, ltw, true);
-          if constexpr (F64) {
-            // W again from its two roots (see col_stage)
-            asm volatile("" : "+v"(x0.x), "+v"(x0.y), "+v"(b1.x), "+v"(b1.y));
-            roots();
-          }
-#pragma unroll
-          for (int m = 0; m < EC; ++m) v[m] = cmul(v[m], W[m]);
-          if (on) {
-#pragma unroll
-            for (int m = 0; m < EC; ++m) st[at + N2 * (t + m * T1)] = v[m];
-          }
+          if (!col_tile<N1, N2, NF, EC, false>(in, a, f, tile, l, on, true, lds, ltw, nle, nls, wait)) return;
         }
-        if (!waited && !wait_team()) return;
+        if (!wait()) return;
         arrive();
       }
     }

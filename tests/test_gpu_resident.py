@@ -159,6 +159,72 @@ def test_wavefront_tiles_give_the_same_bits(gpu, monkeypatch, N, count, ce, conf
     assert all(np.isfinite(f).all() for x in many for f in x if f is not None)
 
 
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("L", [15, 16, 17, 18])
+def test_chip_pass_gives_the_same_bits(gpu, monkeypatch, L, fp32, three):
+    """One instance over all CUs against the stage launches, with both phase sources; NZ of 1 and 2 have no
+    column stage and one."""
+    P = gpu
+    make = c2 if three else c1
+    for NZ, ph in [(5, 0), (5, 1), (2, 0), (1, 0)]:
+        got = []
+        for on in ("1", "0"):
+            monkeypatch.setenv("OPO_RESIDENT", on)
+            got.append(batch_fields(P, [make(N=1 << L, NZ=NZ, NRT=4)], P.FP32C if fp32 else P.FP64, 3,
+                                    col_spt=8, row_spt=8, phase_mode=ph))
+        same(*got)
+
+
+def test_chip_pulsed_instance_and_crystal_pass(gpu, monkeypatch):
+    """EOM and GDD around the whole-chip pass, saved round trips, and the bare crystal pass."""
+    P = gpu
+    outs = []
+    for on in ("1", "0"):
+        monkeypatch.setenv("OPO_RESIDENT", on)
+        one = []
+        for cfg, prec in ((c5(N=1 << 16, NZ=6, NRT=6), P.FP64), (c5(N=1 << 17, NZ=3, NRT=6), P.FP32C)):
+            p, T, w, Ap_in, Ap, As, Ai = inputs(cfg, seed=3, sigma=1e-3)
+            s = P.Solver(P.params_from(P.derive(to_args(cfg)), prec))
+            s.upload(w, T, Ap_in, Ap, As, Ai)
+            s.enable_save(True)
+            s.run(0, 6)
+            one += list(s.download()) + list(s.download_saved().values())
+            s.crystal_pass()
+            one += list(s.download())
+            s.close()
+        outs.append(one)
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
+def test_chip_solvers_side_by_side(gpu):
+    """Large and small solvers on several host threads at once: the whole-chip passes close their teams with the
+    blocks they get beside each other, and every solver gives what it gives alone."""
+    P = gpu
+    cfgs = [c2(N=1 << L, NZ=12, NRT=20) for L in (15, 16, 14, 17, 16, 12)]
+    ins = [inputs(c, seed=70 + k, sigma=1e-3) for k, c in enumerate(cfgs)]
+
+    def one(k, out):
+        p, T, w, Ap_in, Ap, As, Ai = ins[k]
+        s = P.Solver(P.params_from(P.derive(to_args(cfgs[k])), P.FP64))
+        s.upload(w, T, Ap_in, Ap, As, Ai)
+        s.run(0, 20)
+        out[k] = s.download()
+        s.close()
+
+    alone, beside = {}, {}
+    for k in range(len(cfgs)):
+        one(k, alone)
+    th = [threading.Thread(target=one, args=(k, beside)) for k in range(len(cfgs))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for k in range(len(cfgs)):
+        assert all(np.array_equal(a, b) for a, b in zip(alone[k], beside[k])), k
+
+
 def test_noalloc_scratch_holds_as_much_as_without_the_counters(gpu, monkeypatch):
     """The one-launch pass takes its counters from what the scratch has left: the longest power history that the
     scratch holds is the same with and without it, and so are the results just above and below."""
