@@ -113,7 +113,7 @@ struct alignas(128) ResLine {
   unsigned v;
 };
 struct alignas(128) ResLine128 { unsigned v; };
-constexpr int kTeamCounters = 1;
+constexpr int kTeamCounters = 8;
 struct ResTeam {
   ResLine128 part[kTeamCounters];        // stages finished, summed over the team's blocks (block b: part b mod kTeamCounters)
   alignas(128) unsigned long long cur;   // (turn << 32) | instance the team works on
