@@ -157,6 +157,10 @@ struct Engine {
   std::vector<std::pair<int, int>> where;  // batch index -> (group, slot)
 
   hipEvent_t fork_ev = nullptr;
+  // pinned memory that a batch's results pass through (stage_buffer)
+  void *h_stage = nullptr;
+  size_t h_stage_bytes = 0;
+  std::mutex stage_mu;
 
   ~Engine() {
     // release on the engine's device (the caller's current device may differ),
@@ -172,6 +176,7 @@ struct Engine {
       if (g.gs) (void)hipStreamDestroy(g.gs);
     }
     if (fork_ev) (void)hipEventDestroy(fork_ev);
+    if (h_stage) (void)hipHostFree(h_stage);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream && own_stream) (void)hipStreamDestroy(stream);
@@ -234,6 +239,76 @@ int download_c(Engine &E, Group &g, cd *dst, const void *src, size_t n) {
     for (size_t i = 0; i < n; ++i) dst[i] = cd(tmp[2 * i], tmp[2 * i + 1]);
   } else {
     HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(cd), hipMemcpyDeviceToHost, E.stream));
+    HIPCHK(hipStreamSynchronize(E.stream));
+  }
+  return OPO_OK;
+}
+
+// The fields of one instance to the caller's arrays (null: not wanted).  With
+// `conv`, the snapshot if the device's *conv >= 0, else the state.
+//
+// A batch reads instance after instance, so from kStageFrom instances on it
+// keeps pinned memory: one kernel picks the source and writes it there, and
+// the host converts straight into the caller's arrays (4096 samples in FP32C
+// 43 -> 28 us an instance, 2^14 in FP64 88 -> 65; pinning once costs a few
+// hundred us, which a few downloads would not earn back).  Otherwise the
+// copies go to the caller's arrays without a buffer between.
+constexpr int kStageFrom = 16;
+
+// `bytes` of pinned memory, or null (the caller then does without); E.stage_mu is held
+void *stage_buffer(Engine &E, size_t bytes) {
+  if (E.count < kStageFrom) return nullptr;
+  if (E.h_stage_bytes < bytes) {
+    if (E.h_stage) (void)hipHostFree(E.h_stage);
+    E.h_stage = nullptr; E.h_stage_bytes = 0;
+    if (hipHostMalloc(&E.h_stage, bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      E.h_stage = nullptr;
+      return nullptr;
+    }
+    E.h_stage_bytes = bytes;
+  }
+  return E.h_stage;
+}
+
+void widen(double *dst, const float *src, size_t n) {
+  for (size_t i = 0; i < n; ++i) dst[i] = src[i];
+}
+
+int fields_to_host(Engine &E, Group &g, const void *state, const void *snap, const int *conv, double *Ap, double *As,
+                   double *Ai) {
+  double *out[3] = {Ap, As, g.NF == 3 ? Ai : nullptr};
+  const size_t one = (size_t)g.N * esize(g);
+  size_t most = 0;
+  for (const auto &h : E.groups) most = std::max(most, (size_t)h.NF * h.N * esize(h));
+  std::lock_guard<std::mutex> lock(E.stage_mu);
+  if (char *st = static_cast<char *>(stage_buffer(E, most))) {
+    const int e = opo::launch_export(st, state, snap, conv, (long long)(g.NF * one / 16), E.stream);
+    if (e != 0) return fail(OPO_ERR_HIP, std::string("export: ") + hipGetErrorString((hipError_t)e));
+    HIPCHK(hipStreamSynchronize(E.stream));
+    for (int f = 0; f < g.NF; ++f) {
+      if (!out[f]) continue;
+      if (g.fp32) widen(out[f], reinterpret_cast<const float *>(st + f * one), 2 * (size_t)g.N);
+      else std::memcpy(out[f], st + f * one, one);
+    }
+    return OPO_OK;
+  }
+  const void *src = state;
+  if (conv && snap) {
+    int c = -1;
+    HIPCHK(hipMemcpy(&c, conv, sizeof(int), hipMemcpyDeviceToHost));
+    if (c >= 0) src = snap;
+  }
+  const char *from = static_cast<const char *>(src);
+  if (g.fp32) {
+    const std::unique_ptr<float[]> tmp(new float[2 * (size_t)g.NF * g.N]);
+    HIPCHK(hipMemcpyAsync(tmp.get(), from, g.NF * one, hipMemcpyDeviceToHost, E.stream));
+    HIPCHK(hipStreamSynchronize(E.stream));
+    for (int f = 0; f < g.NF; ++f)
+      if (out[f]) widen(out[f], tmp.get() + 2 * (size_t)f * g.N, 2 * (size_t)g.N);
+  } else {
+    for (int f = 0; f < g.NF; ++f)
+      if (out[f]) HIPCHK(hipMemcpyAsync(out[f], from + f * one, one, hipMemcpyDeviceToHost, E.stream));
     HIPCHK(hipStreamSynchronize(E.stream));
   }
   return OPO_OK;
@@ -1269,13 +1344,27 @@ int opo_set_fields(opo_solver *s, const double *Ap, const double *As, const doub
   Engine &E = s->E;
   Group &g = E.groups[0];
   if (!g.inst[0].uploaded) return fail(OPO_ERR_STATE, "set_fields before upload");
-  std::vector<cd> st((size_t)g.NF * g.N, cd(0, 0));
-  for (int j = 0; j < g.N; ++j) {
-    if (Ap) st[j] = cd(Ap[2 * j], Ap[2 * j + 1]);
-    if (As) st[(size_t)g.N + j] = cd(As[2 * j], As[2 * j + 1]);
-    if (g.NF == 3 && Ai) st[(size_t)2 * g.N + j] = cd(Ai[2 * j], Ai[2 * j + 1]);
+  // straight from the caller's arrays, without a copy of all three between
+  const double *in[3] = {Ap, As, Ai};
+  const size_t one = (size_t)g.N * esize(g);
+  const std::unique_ptr<float[]> tmp(g.fp32 ? new float[2 * (size_t)g.NF * g.N] : nullptr);
+  for (int f = 0; f < g.NF; ++f) {
+    char *dst = static_cast<char *>(g.inst[0].state) + f * one;
+    if (!in[f]) {
+      const int e = opo::launch_zero(dst, (long long)(one / 8), E.stream);
+      if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
+      continue;
+    }
+    const void *src = in[f];
+    if (g.fp32) {
+      float *t = tmp.get() + 2 * (size_t)f * g.N;
+      for (size_t j = 0; j < 2 * (size_t)g.N; ++j) t[j] = (float)in[f][j];
+      src = t;
+    }
+    HIPCHK(hipMemcpyAsync(dst, src, one, hipMemcpyHostToDevice, E.stream));
   }
-  return upload_c(E, g, g.inst[0].state, st.data(), st.size());
+  HIPCHK(hipStreamSynchronize(E.stream));
+  return OPO_OK;
 }
 
 namespace {
@@ -1482,12 +1571,7 @@ int opo_download(opo_solver *s, double *Ap, double *As, double *Ai) {
   HIPCHK(hipSetDevice(s->E.device));
   Engine &E = s->E;
   Group &g = E.groups[0];
-  std::vector<cd> st((size_t)g.NF * g.N);
-  RCHK(download_c(E, g, st.data(), g.inst[0].state, st.size()));
-  if (Ap) std::memcpy(Ap, st.data(), g.N * sizeof(cd));
-  if (As) std::memcpy(As, st.data() + g.N, g.N * sizeof(cd));
-  if (Ai && g.NF == 3) std::memcpy(Ai, st.data() + 2 * (size_t)g.N, g.N * sizeof(cd));
-  return OPO_OK;
+  return fields_to_host(E, g, g.inst[0].state, nullptr, nullptr, Ap, As, Ai);
 }
 
 int opo_download_saved(opo_solver *s, double *sp, double *ss, double *si) {
@@ -1778,15 +1862,7 @@ int opo_batch_download(opo_batch *b, int idx, double *Ap, double *As, double *Ai
   Engine &E = b->E;
   auto [gi, k] = E.where[idx];
   Group &g = E.groups[gi];
-  int conv = -1;
-  HIPCHK(hipMemcpy(&conv, g.d_conv + k, sizeof(int), hipMemcpyDeviceToHost));
-  const void *src = (conv >= 0 && g.inst[k].snap) ? g.inst[k].snap : g.inst[k].state;
-  std::vector<cd> st((size_t)g.NF * g.N);
-  RCHK(download_c(E, g, st.data(), src, st.size()));
-  if (Ap) std::memcpy(Ap, st.data(), g.N * sizeof(cd));
-  if (As) std::memcpy(As, st.data() + g.N, g.N * sizeof(cd));
-  if (Ai && g.NF == 3) std::memcpy(Ai, st.data() + 2 * (size_t)g.N, g.N * sizeof(cd));
-  return OPO_OK;
+  return fields_to_host(E, g, g.inst[k].state, g.inst[k].snap, g.d_conv + k, Ap, As, Ai);
 }
 
 int opo_batch_power_history(opo_batch *b, int idx, double *out, int n) {
@@ -1804,15 +1880,16 @@ int opo_batch_power(opo_batch *b, double *out) {
   if (!b || !out) return fail(OPO_ERR_INVALID, "null");
   HIPCHK(hipSetDevice(b->E.device));
   Engine &E = b->E;
+  std::lock_guard<std::mutex> lock(E.stage_mu);
   for (auto &g : E.groups) {
     const int n = (int)g.members.size();
-    std::vector<int> rt(n);
-    HIPCHK(hipMemcpy(rt.data(), g.d_rt, n * sizeof(int), hipMemcpyDeviceToHost));
-    for (int k = 0; k < n; ++k) {
-      const int last = std::max(0, std::min(rt[k], g.hist_len) - 1);
-      HIPCHK(hipMemcpy(out + g.members[k], g.d_hist + (size_t)k * g.hist_len + last, sizeof(double),
-                       hipMemcpyDeviceToHost));
-    }
+    // every instance's last power in one copy, through the (idle) partials
+    const int e = opo::launch_last_power(g.d_partials, g.d_hist, g.d_rt, g.hist_len, n, E.stream);
+    if (e != 0) return fail(OPO_ERR_HIP, std::string("power: ") + hipGetErrorString((hipError_t)e));
+    std::vector<double> last(n);
+    HIPCHK(hipMemcpyAsync(last.data(), g.d_partials, n * sizeof(double), hipMemcpyDeviceToHost, E.stream));
+    HIPCHK(hipStreamSynchronize(E.stream));
+    for (int k = 0; k < n; ++k) out[g.members[k]] = last[k];
   }
   return OPO_OK;
 }

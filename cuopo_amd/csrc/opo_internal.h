@@ -194,6 +194,8 @@ int launch_accel_dots(int fp32, const AccelDesc *d, int count, int nres, long lo
 int launch_accel_apply(int fp32, const AccelDesc *d, int count, int nres, long long N, void *stream);
 // zero fill of `words` 8-byte words on `stream`
 int launch_zero(void *dst, long long words, void *stream);
+int launch_export(void *pinned, const void *state, const void *snap, const int *conv, long long words16, void *stream);
+int launch_last_power(double *out, const double *hist, const int *rt, int hist_len, int n, void *stream);
 
 // The no-allocation entry point's device memory: a static array of
 // kScratchBytes per GPU (opo_kernels.hip).  scratch_region returns the

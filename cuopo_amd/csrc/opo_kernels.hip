@@ -840,6 +840,37 @@ int launch_zero(void *dst, long long words, void *stream) {
   return (int)hipGetLastError();
 }
 
+// One instance's fields into pinned host memory, from the snapshot where there
+// is one and *conv >= 0, else from the state (opo_batch_download): a launch
+// in place of a copy of the flag, a wait and a copy of the fields.  Bound by
+// the host link; 16 bytes a thread.
+__global__ __launch_bounds__(256) void export_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ state,
+                                                     const uint4 *__restrict__ snap, const int *__restrict__ conv,
+                                                     long long n) {
+  const uint4 *src = snap && conv && *conv >= 0 ? snap : state;
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
+int launch_export(void *pinned, const void *state, const void *snap, const int *conv, long long words16, void *stream) {
+  hipLaunchKernelGGL(export_kernel, dim3((unsigned)((words16 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                     (uint4 *)pinned, (const uint4 *)state, (const uint4 *)snap, conv, words16);
+  return (int)hipGetLastError();
+}
+
+// every instance's power after its last round trip (one copy to the host
+// instead of one per instance: 256 of them 3.3 -> 0.07 ms)
+__global__ __launch_bounds__(256) void last_power(double *__restrict__ out, const double *__restrict__ hist,
+                                                  const int *__restrict__ rt, int hist_len, int n) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) out[k] = hist[(long long)k * hist_len + max(0, min(rt[k], hist_len) - 1)];
+}
+
+int launch_last_power(double *out, const double *hist, const int *rt, int hist_len, int n, void *stream) {
+  hipLaunchKernelGGL(last_power, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, out, hist, rt, hist_len, n);
+  return (int)hipGetLastError();
+}
+
 // ------------------------------------------------ no-allocation scratch
 // Device memory of the no-allocation entry point: one array of kScratchBytes
 // per GPU, loaded with the code object and held until the process ends.  In
