@@ -670,9 +670,10 @@ ResShape res_shape(const Engine &E, const Group &g) { return res_shape(g, res_co
 constexpr long long kResTurn = 1LL << 19;  // samples of one turn of every XCD's teams
 constexpr double kResTurnUs = 16.5, kStreamUs = 7.0, kStreamUsPerSample = 31e-6;
 
-// One instance of 2^15 samples or more with 8 samples per thread: the whole
-// chip works on it (opo_chip.h: 1.2 to 1.4 times the two-launch path, 1.1
-// times one XCD's team at 2^15).  Below, rows no longer fill a wavefront and
+// One instance of 2^15 samples or more with 8 samples per thread in the rows:
+// the whole chip works on it (opo_chip.h: 1.15 to 1.45 times the two-launch
+// path at the same settings, 1.1 times one XCD's team at 2^15, with 4 samples
+// per thread in the columns 1.7 times).  Below, rows no longer fill a wavefront and
 // one XCD's barrier is the cheaper one (2^14: 7.0 us a slice); several
 // instances fill the chip stage by stage.
 bool chip_wide(const Engine &E, const Group &g) {
@@ -725,7 +726,7 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   a.sync = g.d_sync;
   a.err = g.d_err;
   if (chip_wide(E, g)) {
-    const int e = opo::launch_chip(g.fp32, g.N1, g.N2, g.NF, g.d_insts, a, g.cur);
+    const int e = opo::launch_chip(g.fp32, g.N1, g.N2, g.NF, g.ce, g.d_insts, a, g.cur);
     if (e != 0) return fail(OPO_ERR_HIP, std::string("chip pass launch: ") + hipGetErrorString((hipError_t)e));
     return OPO_OK;
   }

@@ -9,10 +9,12 @@
 // keeps to one block.  Per slice, two-launch -> this, three equations: 2^15
 // 10.2 -> 8.5 us FP64, 9.9 -> 8.0 FP32C (one XCD's team: 9.4 FP64); 2^16 13.3
 // -> 9.7, 11.7 -> 8.6; 2^17 17.7 -> 13.0, 14.7 -> 10.3; 2^18 28.5 -> 20.7,
-// 20.7 -> 14.7.  What bounds it: a stage at 2^16 is 2.9 us of exchange (below)
-// beside 1.4 to 1.9 us of transforms with one wavefront per SIMD; at 2^18
-// 12.6 MB pass through the fabric twice per stage (3.7 to 4.0 us) beside the
-// transforms (6 us of FP64 on the CUs that hold two of the 384 rows).
+// 20.7 -> 14.7; with 4 samples per thread in the columns 10.4 -> 7.6 at 2^15,
+// 13.3 -> 9.6 at 2^16, 28.9 -> 25.2 at 2^18 (FP64).  What bounds it: a stage
+// at 2^16 is 2.9 us of exchange (below) beside 1.4 to 1.9 us of transforms
+// with one wavefront per SIMD; at 2^18 12.6 MB pass through the fabric twice
+// per stage (3.7 to 4.0 us) beside the transforms (4 us of FP64 on the CUs
+// that hold two of the 384 rows).
 //
 // Memory order.  Blocks read what other XCDs wrote, so the fields are stored at
 // agent scope as well as loaded (sc1: past the XCD's L2); a block waits for its
@@ -213,6 +215,14 @@ int launch_chip_k(const OpoInst *insts, ResArgs a, hipStream_t s) {
   a.expect = grid;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, insts, a);
   return (int)hipGetLastError();
+}
+
+// 8 samples per thread in rows (with 4 their teams would not fit a block), 8 or 4 in columns
+template <typename T, int N1, int N2>
+int launch_chip_n(int NF, int ce, const OpoInst *insts, const ResArgs &a, hipStream_t s) {
+  if (ce == 8)
+    return NF == 3 ? launch_chip_k<T, N1, N2, 3, 8, 8>(insts, a, s) : launch_chip_k<T, N1, N2, 2, 8, 8>(insts, a, s);
+  return NF == 3 ? launch_chip_k<T, N1, N2, 3, 4, 8>(insts, a, s) : launch_chip_k<T, N1, N2, 2, 4, 8>(insts, a, s);
 }
 
 }  // namespace opo

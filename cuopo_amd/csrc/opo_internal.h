@@ -143,7 +143,7 @@ bool resident_supported(int N1, int N2, int ce, int re);
 constexpr int kChipBlocks = 256;  // one per CU
 constexpr int kChipCounters = 64;
 bool chip_supported(int N1, int N2, int ce, int re, int fp32);
-int launch_chip(int fp32, int N1, int N2, int NF, const OpoInst *insts, const ResArgs &a, void *stream);
+int launch_chip(int fp32, int N1, int N2, int NF, int ce, const OpoInst *insts, const ResArgs &a, void *stream);
 int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoInst *insts, const ResArgs &a, int grid,
                     void *stream);
 

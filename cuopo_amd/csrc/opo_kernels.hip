@@ -737,17 +737,17 @@ int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoI
   return f(N1, N2, ce, re, insts, a, grid, (hipStream_t)stream);
 }
 
-// One instance of N = 2^16 .. 2^18 over all CUs (opo_chip_*.hip), 8 samples per thread.
-int launch_chip_f64(int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
-int launch_chip_f32(int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
+// One instance of N = 2^16 .. 2^18 over all CUs (opo_chip_*.hip), 8 samples per thread in the rows.
+int launch_chip_f64(int, int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
+int launch_chip_f32(int, int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
 
 bool chip_supported(int N1, int N2, int ce, int re, int fp32) {
-  if (ce != 8 || re != 8) return false;
+  if ((ce != 8 && ce != 4) || re != 8) return false;
   return (N1 == 64 && (N2 == 512 || N2 == 1024 || N2 == 2048)) || (fp32 ? N1 == 64 && N2 == 4096 : N1 == 128 && N2 == 2048);
 }
 
-int launch_chip(int fp32, int N1, int N2, int NF, const OpoInst *insts, const ResArgs &a, void *stream) {
-  return (fp32 ? launch_chip_f32 : launch_chip_f64)(N1, N2, NF, insts, a, (hipStream_t)stream);
+int launch_chip(int fp32, int N1, int N2, int NF, int ce, const OpoInst *insts, const ResArgs &a, void *stream) {
+  return (fp32 ? launch_chip_f32 : launch_chip_f64)(N1, N2, NF, ce, insts, a, (hipStream_t)stream);
 }
 
 // ------------------------------------------------ round-trip extrapolation

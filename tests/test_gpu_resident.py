@@ -167,12 +167,12 @@ def test_chip_pass_gives_the_same_bits(gpu, monkeypatch, L, fp32, three):
     column stage and one."""
     P = gpu
     make = c2 if three else c1
-    for NZ, ph in [(5, 0), (5, 1), (2, 0), (1, 0)]:
+    for NZ, ph, ce in [(5, 0, 8), (5, 1, 8), (2, 0, 8), (1, 0, 8), (3, 0, 4)]:
         got = []
         for on in ("1", "0"):
             monkeypatch.setenv("OPO_RESIDENT", on)
             got.append(batch_fields(P, [make(N=1 << L, NZ=NZ, NRT=4)], P.FP32C if fp32 else P.FP64, 3,
-                                    col_spt=8, row_spt=8, phase_mode=ph))
+                                    col_spt=ce, row_spt=8, phase_mode=ph))
         same(*got)
 
 
