@@ -104,8 +104,7 @@ __global__ __launch_bounds__((chip_threads<N1, N2, NF, EC, ER>())) void chip_pas
           at += nx[i];
         }
       }
-      if (poll_until(&S->size[x].v, [](unsigned v) { return v != 0; })) word = agent_load(&S->size[x].v);
-      else agent_store(&a.err[0], 1);
+      if (!poll_until(&S->size[x].v, [](unsigned v) { return v != 0; }, &word)) agent_store(&a.err[0], 1);
     }
     sh_rank = old;
     sh_word = word;

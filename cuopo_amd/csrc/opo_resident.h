@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "opo_device.h"
+#include "opo_handoff.h"
 #include "opo_internal.h"
 
 namespace opo {
@@ -58,14 +59,29 @@ template <typename T> __device__ __forceinline__ void agent_store(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Polls until f(value) holds; false on a time-out.
-template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *p, F f) {
+// Polls until f(value) holds, then *got is that value; false on a time-out.
+template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *p, F f, T *got) {
   for (unsigned n = 0; n < kMaxPolls; ++n) {
-    if (f(agent_load(p))) return true;
+    const T v = agent_load(p);
+    if (f(v)) {
+      *got = v;
+      return true;
+    }
     __builtin_amdgcn_s_sleep(1);
   }
   return false;
 }
+
+// The launch's queue and a team's word, for hand_out and hand_in.
+struct TeamQueue {
+  ResSync *S;
+  ResTeam *tm;
+  __device__ __forceinline__ unsigned take() { return agent_add(&S->next.v, 1u); }
+  __device__ __forceinline__ void publish(unsigned long long w) { agent_store(&tm->cur, w); }
+  __device__ __forceinline__ bool await(unsigned turn, unsigned long long *w) {
+    return poll_until(&tm->cur, [turn](unsigned long long v) { return is_turn(v, turn); }, w);
+  }
+};
 
 // Coherent loads of the instance's fields: 16- (8-) byte buffer loads at agent
 // scope.  `off` in elements.
@@ -268,7 +284,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
   constexpr unsigned N = N1 * N2;
   static_assert(T1 <= 64 && T2 <= 64 && NTC >= 1 && NTR >= 1, "one wavefront per field");
   extern __shared__ __align__(16) unsigned char smem_raw[];  // (the static words before it are not a multiple of 16 bytes)
-  __shared__ unsigned long long sh_next[2];
+  __shared__ unsigned sh_next[2];
   __shared__ int sh_rank, sh_size, sh_ok;
   V *ltw = reinterpret_cast<V *>(smem_raw);  // N1-point root table
   const int tid = threadIdx.x;
@@ -292,11 +308,12 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
       size = (int)__hip_atomic_fetch_or(&S->join[x].v, kTeamClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       agent_store(&S->size[x].v, (unsigned)size);
     } else {
-      if (!poll_until(&S->size[x].v, [](unsigned v) { return v != 0; })) {
+      unsigned closed = 0;
+      if (!poll_until(&S->size[x].v, [](unsigned v) { return v != 0; }, &closed)) {
         agent_store(&a.err[0], 1);
         size = -1;
       } else {
-        size = (int)agent_load(&S->size[x].v);
+        size = (int)closed;
       }
     }
     sh_rank = (int)old;
@@ -318,12 +335,15 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
   const int size = min(per, xs - team * per);
   ResTeam *tm = &S->team[team * kXcds + x];
   const int nsub = a.sub, workers = size * nsub;
+  const unsigned total = (unsigned)(a.count + a.count2);
+  TeamQueue queue{S, tm};
+  auto inst = [&](unsigned i) { return i < (unsigned)a.count ? insts + i : a.insts2 + (i - (unsigned)a.count); };
   unsigned arrived = 0;  // stages finished
 
   for (unsigned epoch = 1;; ++epoch) {
     // ---- the team's next instance ----
     if (tid == 0) {
-      unsigned long long w = 0;
+      unsigned i = ~0u;
       if (r0 == 0) {
         if (epoch == 1 && a.spread) {
           // fewer instances than teams: each launch prefers an XCD of its own,
@@ -333,20 +353,16 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
           while (wall_clock64() - t0 < d) {
           }
         }
-        w = ((unsigned long long)epoch << 32) | agent_add(&S->next.v, 1u);
-        agent_store(&tm->cur, w);
-      } else {
-        const bool ok = poll_until(&tm->cur, [epoch](unsigned long long v) { return (unsigned)(v >> 32) == epoch; });
-        w = ok ? agent_load(&tm->cur) : ~0ull;
-        if (!ok) agent_store(&a.err[0], 2);
+        i = hand_out(queue, epoch, total, [&](unsigned k) { return inst(k)->active_v != 0; });
+      } else if (!hand_in(queue, epoch, &i)) {
+        agent_store(&a.err[0], 2);  // (i stays past the end: the block leaves)
       }
-      sh_next[epoch & 1] = w;
+      sh_next[epoch & 1] = i;
     }
     __syncthreads();
-    const unsigned idx = __builtin_amdgcn_readfirstlane((unsigned)sh_next[epoch & 1]);
-    if (idx >= (unsigned)(a.count + a.count2)) return;
-    const auto I = cp_scalar(idx < (unsigned)a.count ? insts + idx : a.insts2 + (idx - (unsigned)a.count));
-    if (I->active_v == 0) continue;
+    const unsigned idx = __builtin_amdgcn_readfirstlane(sh_next[epoch & 1]);
+    if (idx >= total) return;
+    const auto I = cp_scalar(inst(idx));
     V *state = reinterpret_cast<V *>(I->state);
     const FieldBuf<V> in(state, NF * N * (unsigned)sizeof(V));
     const double *nl = I->nl;
@@ -419,6 +435,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
         arrive();
       }
     }
+    if (ends_with_wait(a.NZ) && !wait_team()) return;
   }
 }
 
