@@ -760,8 +760,10 @@ int check_resident(Engine &E) {
 // two of 2^18 23.7 -> 17.7; below, the thinner launch loses: 62 of 2^12 (496
 // wavefronts) 13.2 -> 13.4, eight of 2^14 (256) 8.5 -> 10.7.  FP32C gains from
 // a few more on: 64 of 2^14 20.6 -> 16.1, 62 of 2^13 (992) 14.0 -> 13.9, 128 of
-// 2^12 (1024) 13.4 -> 13.6.
+// 2^12 (1024) 13.4 -> 13.6.  A tile is 64 * ce / N1 columns of all rows; at 2^8
+// with 8 samples per thread that is 32 of 16 columns, so those stay per field.
 bool wave_tiles(const Group &g) {
+  if (64 * g.ce / g.N1 > g.N2) return false;
   const long long waves = (long long)g.launch_n * g.N / (64 * g.ce);
   return waves >= (g.fp32 ? 1100 : 960);
 }
