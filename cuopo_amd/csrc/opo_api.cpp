@@ -136,6 +136,7 @@ struct Engine {
   int accel_every = 0;     // round-trip extrapolation every this many round trips (0: off), see accel_step
   int accel_start = 1000;  // ... from this many round trips of the run on
   bool resident = true;  // crystal passes as one launch where every group allows it (opo_resident.h)
+  unsigned polls = opo::kMaxPolls;  // after which a wait of such a pass gives up
   bool timing = false;   // the autotuner is timing slices
   bool forked = false;   // the groups' chains run on their own streams (fork_groups .. join_groups)
   bool save_enabled = false;
@@ -369,6 +370,16 @@ int check_shapes(const Group &g) {
   if (g.N1 < 16 || g.N2 < 16 || g.N1 > 128 || g.N2 > 4096 || (long long)g.N1 * g.N2 != g.N)
     return fail(OPO_ERR_INVALID, "internal: four-step split out of range");
   return OPO_OK;
+}
+
+// OPO_RESIDENT=0 launches every stage of a crystal pass by itself;
+// OPO_RESIDENT_POLLS sets after how many reads a wait of a one-launch pass
+// gives up (the call then returns an error).
+void read_resident_env(Engine &E) {
+  if (const char *rs = std::getenv("OPO_RESIDENT")) E.resident = rs[0] != '0';
+  const char *rp = std::getenv("OPO_RESIDENT_POLLS");
+  if (rp && *rp)
+    E.polls = (unsigned)std::min<unsigned long>(std::strtoul(rp, nullptr, 10), opo::kMaxPolls);
 }
 
 // Counters of the one-launch crystal passes.  In the no-allocation mode they
@@ -723,6 +734,7 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   a.spread = total < r.teams * opo::kXcds;
   // consecutive handles prefer different XCDs
   a.prefer = (int)((reinterpret_cast<uintptr_t>(g.d_insts) >> 12) % opo::kXcds);
+  a.polls = E.polls;
   a.sync = g.d_sync;
   a.err = g.d_err;
   if (chip_wide(E, g)) {
@@ -735,20 +747,22 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   return OPO_OK;
 }
 
-// A pass whose blocks waited too long for each other left its fields undefined.
+// A pass whose blocks waited too long for each other left its fields
+// undefined.  The flags are clear again afterwards, so that an error is
+// reported by the call it happened in and by no other.
 int check_resident(Engine &E) {
+  bool timed_out = false;
   for (auto &g : E.groups) {
     if (!g.d_err) continue;
     int err = 0;
     HIPCHK(hipMemcpyAsync(&err, g.d_err, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     HIPCHK(hipStreamSynchronize(E.stream));
-    if (err != 0) {
-      const int e = opo::launch_zero(g.d_err, 1, E.stream);
-      if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
-      return fail(OPO_ERR_HIP, "crystal pass timed out on the device");
-    }
+    if (err == 0) continue;
+    timed_out = true;
+    const int e = opo::launch_zero(g.d_err, 1, E.stream);
+    if (e != 0) return fail(OPO_ERR_HIP, std::string("zero fill: ") + hipGetErrorString((hipError_t)e));
   }
-  return OPO_OK;
+  return timed_out ? fail(OPO_ERR_HIP, "crystal pass timed out on the device") : OPO_OK;
 }
 
 // ------------------------------------------------------------ stage emitters
@@ -1243,8 +1257,7 @@ int engine_init(Engine &E, const opo_params *params, int count) {
   // OPO_SPLIT=0 keeps a large one-grid batch in one group (see split_large_group)
   bool split = true;
   if (const char *sp = std::getenv("OPO_SPLIT")) split = sp[0] != '0';
-  // OPO_RESIDENT=0 launches every stage of a crystal pass by itself
-  if (const char *rs = std::getenv("OPO_RESIDENT")) E.resident = rs[0] != '0';
+  read_resident_env(E);
   E.count = count; E.NZ = p0.NZ; E.three_eqs = p0.three_eqs ? 1 : 0; E.regime = p0.regime;
   E.fp32 = p0.precision == OPO_FP32C; E.device = p0.device;
   E.NRT = 1;
@@ -1558,7 +1571,7 @@ int opo_run_noalloc(const opo_params *params, const double *w, const double *T, 
   RCHK(make_group(E, g));
   g.inst[0].prm = *params;
   RCHK(upload_instance(E, g, 0, w, T, nullptr, n_ap, nullptr, nullptr, nullptr));
-  if (const char *rs = std::getenv("OPO_RESIDENT")) E.resident = rs[0] != '0';
+  read_resident_env(E);
   RCHK(alloc_sync(E, g));  // last: it never takes what the instance needs
   RCHK(engine_run(E, rt0, n_rt, 0, 0.0));
   if (power_out) {
@@ -1684,6 +1697,7 @@ int engine_time_slices(Engine &E, Group &g, int iters, double *slice_us) {
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc != OPO_OK) return rc;
+  RCHK(check_resident(E));
   *slice_us = 1e3 * ms / iters;
   return OPO_OK;
 }
@@ -1722,6 +1736,7 @@ int engine_time_joint(Engine &E, int iters, double *slice_us) {
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc != OPO_OK) return rc;
+  RCHK(check_resident(E));
   *slice_us = 1e3 * ms / iters;
   return OPO_OK;
 }
@@ -2055,7 +2070,7 @@ int autotune_joint(Engine &E, int iters) {
 // column settings, then the column settings once more beside those rows.
 // With several grid sizes, autotune_joint then weighs the picks side by side.
 // The timed slices mutate the fields, so each group's state is saved before
-// and restored after.
+// and restored after, as are the settings if the tuning fails.
 int engine_autotune(Engine &E, int iters) {
   for (size_t gi = 0; gi < E.groups.size(); ++gi) {
     Group &g = E.groups[gi];
@@ -2083,6 +2098,8 @@ int engine_autotune(Engine &E, int iters) {
     HIPCHK(hipStreamSynchronize(E.stream));
     opo_tuning base;
     get_tuning(E, g, &base);
+    opo_tuning before = base;  // as set_tuning has it: 0 and -1 stay "as the engine's"
+    before.col_threads = g.col_threads; before.row_threads = g.row_threads; before.xcd_pack = g.xcd_pack;
     const int ct0 = (int)(128 / esize(g));
     std::vector<int> xcds = {0};
     if ((long long)n * g.N <= (1LL << 16)) xcds.push_back(1);
@@ -2126,37 +2143,43 @@ int engine_autotune(Engine &E, int iters) {
         }
       return OPO_OK;
     };
-    for (int x : xcds) {
-      opo_tuning t = base;
-      t.xcd_pack = x;
-      t.row_threads = 64; t.row_spt = 8; t.phase_mode = -1;
-      double bc = 1e30;
-      opo_tuning tc = t;
-      RCHK(col_pass(t, &tc, &bc));
-      double br = 1e30;
-      opo_tuning tr = tc;
-      for (int spt : {8, 4})
-        for (int r : rts)
-          for (int ph : phases) {
-            opo_tuning c = tc;
-            c.row_threads = r; c.row_spt = spt; c.phase_mode = ph;
-            double us = 0;
-            const int rc = time_it(c, &us);
-            if (rc < 0) return rc;
-            if (rc == OPO_OK && us < br) { br = us; tr = c; }
-          }
-      // the column settings again, now beside the chosen rows: the first pass
-      // ranked them beside default rows, and a column tile's neighbour in the
-      // slice can change its rank
-      const opo_tuning rows = tr;
-      RCHK(col_pass(rows, &tr, &br));
-      if (br < best_us) { best_us = br; best = tr; }
-    }
-    RCHK(set_tuning(E, g, &best));
-    g.tuned_us = best_us;
+    auto tune = [&]() -> int {
+      for (int x : xcds) {
+        opo_tuning t = base;
+        t.xcd_pack = x;
+        t.row_threads = 64; t.row_spt = 8; t.phase_mode = -1;
+        double bc = 1e30;
+        opo_tuning tc = t;
+        RCHK(col_pass(t, &tc, &bc));
+        double br = 1e30;
+        opo_tuning tr = tc;
+        for (int spt : {8, 4})
+          for (int r : rts)
+            for (int ph : phases) {
+              opo_tuning c = tc;
+              c.row_threads = r; c.row_spt = spt; c.phase_mode = ph;
+              double us = 0;
+              const int rc = time_it(c, &us);
+              if (rc < 0) return rc;
+              if (rc == OPO_OK && us < br) { br = us; tr = c; }
+            }
+        // the column settings again, now beside the chosen rows: the first pass
+        // ranked them beside default rows, and a column tile's neighbour in the
+        // slice can change its rank
+        const opo_tuning rows = tr;
+        RCHK(col_pass(rows, &tr, &br));
+        if (br < best_us) { best_us = br; best = tr; }
+      }
+      return OPO_OK;
+    };
+    const int rc = tune();
+    const std::string why = rc == OPO_OK ? "" : g_err;
+    RCHK(set_tuning(E, g, rc == OPO_OK ? &best : &before));
+    g.tuned_us = rc == OPO_OK ? best_us : before.slice_us;
     for (int k = 0; k < n; ++k)
       HIPCHK(hipMemcpyAsync(g.inst[k].state, (char *)bak + bytes * k, bytes, hipMemcpyDeviceToDevice, E.stream));
     HIPCHK(hipStreamSynchronize(E.stream));
+    if (rc != OPO_OK) return fail(rc, why);
   }
   RCHK(autotune_joint(E, iters));
   RCHK(sync_insts(E));

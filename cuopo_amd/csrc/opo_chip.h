@@ -104,7 +104,7 @@ __global__ __launch_bounds__((chip_threads<N1, N2, NF, EC, ER>())) void chip_pas
           at += nx[i];
         }
       }
-      if (!poll_until(&S->size[x].v, [](unsigned v) { return v != 0; }, &word)) agent_store(&a.err[0], 1);
+      if (!poll_until(&S->size[x].v, a.polls, [](unsigned v) { return v != 0; }, &word)) agent_store(&a.err[0], 1);
     }
     sh_rank = old;
     sh_word = word;
@@ -132,7 +132,7 @@ __global__ __launch_bounds__((chip_threads<N1, N2, NF, EC, ER>())) void chip_pas
     if (tid < kChipCounters) {
       const unsigned need = stages * (unsigned)((size + kChipCounters - 1 - tid) / kChipCounters);
       bool ok = false;
-      for (unsigned n = 0; n < kMaxPolls && !ok; ++n) {
+      for (unsigned n = 0; n < a.polls && !ok; ++n) {
         ok = __all((int)(agent_load(&S->team[tid].part[0].v) - need) >= 0);
         if (!ok) __builtin_amdgcn_s_sleep(1);
       }

@@ -133,13 +133,14 @@ struct ResArgs {
   int sub;           // tiles a block works on side by side
   int expect;        // blocks per XCD
   int spread, prefer;  // fewer instances than teams: XCD that takes the first one
-  unsigned zero;     // 0
+  unsigned polls;    // a wait gives up after so many reads
   void *sync;        // ResSync
   int *err;          // set on a time-out, never cleared by a kernel
 };
 // threads per block of the resident pass
 constexpr int res_max_threads(int, int) { return 768; }
 bool resident_supported(int N1, int N2, int ce, int re);
+constexpr unsigned kMaxPolls = 1u << 23;  // seconds: a poll takes a few hundred ns
 constexpr int kChipBlocks = 256;  // one per CU
 constexpr int kChipCounters = 64;
 bool chip_supported(int N1, int N2, int ce, int re, int fp32);

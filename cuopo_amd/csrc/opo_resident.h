@@ -44,7 +44,6 @@ namespace opo {
 
 constexpr unsigned kTeamClosed = 1u << 20;
 constexpr unsigned long long kJoinTicks = 2000;          // 20 us of the 100 MHz clock
-constexpr unsigned kMaxPolls = 1u << 23;                 // seconds: a poll takes a few hundred ns
 
 __device__ __forceinline__ unsigned xcc_id() {
   return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & (kXcds - 1);  // hwreg(HW_REG_XCC_ID, 0, 4)
@@ -59,9 +58,9 @@ template <typename T> __device__ __forceinline__ void agent_store(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Polls until f(value) holds, then *got is that value; false on a time-out.
-template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *p, F f, T *got) {
-  for (unsigned n = 0; n < kMaxPolls; ++n) {
+// Polls until f(value) holds, then *got is that value; false after `polls` reads.
+template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *p, unsigned polls, F f, T *got) {
+  for (unsigned n = 0; n < polls; ++n) {
     const T v = agent_load(p);
     if (f(v)) {
       *got = v;
@@ -76,10 +75,11 @@ template <typename T, typename F> __device__ __forceinline__ bool poll_until(T *
 struct TeamQueue {
   ResSync *S;
   ResTeam *tm;
+  unsigned polls;
   __device__ __forceinline__ unsigned take() { return agent_add(&S->next.v, 1u); }
   __device__ __forceinline__ void publish(unsigned long long w) { agent_store(&tm->cur, w); }
   __device__ __forceinline__ bool await(unsigned turn, unsigned long long *w) {
-    return poll_until(&tm->cur, [turn](unsigned long long v) { return is_turn(v, turn); }, w);
+    return poll_until(&tm->cur, polls, [turn](unsigned long long v) { return is_turn(v, turn); }, w);
   }
 };
 
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
       agent_store(&S->size[x].v, (unsigned)size);
     } else {
       unsigned closed = 0;
-      if (!poll_until(&S->size[x].v, [](unsigned v) { return v != 0; }, &closed)) {
+      if (!poll_until(&S->size[x].v, a.polls, [](unsigned v) { return v != 0; }, &closed)) {
         agent_store(&a.err[0], 1);
         size = -1;
       } else {
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
   ResTeam *tm = &S->team[team * kXcds + x];
   const int nsub = a.sub, workers = size * nsub;
   const unsigned total = (unsigned)(a.count + a.count2);
-  TeamQueue queue{S, tm};
+  TeamQueue queue{S, tm, a.polls};
   auto inst = [&](unsigned i) { return i < (unsigned)a.count ? insts + i : a.insts2 + (i - (unsigned)a.count); };
   unsigned arrived = 0;  // stages finished
 
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
         const int c = lane & (kTeamCounters - 1);
         const unsigned need = arrived * (unsigned)((size + kTeamCounters - 1 - c) / kTeamCounters);
         bool ok = false;
-        for (unsigned n = 0; n < kMaxPolls && !ok; ++n) {
+        for (unsigned n = 0; n < a.polls && !ok; ++n) {
           ok = lane >= kTeamCounters || (int)(agent_load(&tm->part[c].v) - need) >= 0;
           ok = __all(ok);
           if (!ok) __builtin_amdgcn_s_sleep(1);
