@@ -735,6 +735,7 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   // consecutive handles prefer different XCDs
   a.prefer = (int)((reinterpret_cast<uintptr_t>(g.d_insts) >> 12) % opo::kXcds);
   a.polls = E.polls;
+  a.always = E.solver;
   a.sync = g.d_sync;
   a.err = g.d_err;
   if (chip_wide(E, g)) {

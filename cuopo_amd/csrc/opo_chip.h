@@ -121,7 +121,7 @@ __global__ __launch_bounds__((chip_threads<N1, N2, NF, EC, ER>())) void chip_pas
   unsigned *mine_cnt = &S->team[rank & (kChipCounters - 1)].part[0].v;
 
   const auto I = cp_scalar(insts);
-  if (I->active_v == 0) return;
+  if (!a.always && I->active_v == 0) return;
   const FieldBuf<V> in(reinterpret_cast<V *>(I->state), NF * N * (unsigned)sizeof(V));
   const double *nl = I->nl;
   const double h6 = I->h6;

@@ -134,6 +134,7 @@ struct ResArgs {
   int expect;        // blocks per XCD
   int spread, prefer;  // fewer instances than teams: XCD that takes the first one
   unsigned polls;    // a wait gives up after so many reads
+  int always;        // a solver's instance: run whatever its descriptor says, as the stages' direct kernels do
   void *sync;        // ResSync
   int *err;          // set on a time-out, never cleared by a kernel
 };

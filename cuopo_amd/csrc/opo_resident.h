@@ -353,7 +353,7 @@ __global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const O
           while (wall_clock64() - t0 < d) {
           }
         }
-        i = hand_out(queue, epoch, total, [&](unsigned k) { return inst(k)->active_v != 0; });
+        i = hand_out(queue, epoch, total, [&](unsigned k) { return a.always || inst(k)->active_v != 0; });
       } else if (!hand_in(queue, epoch, &i)) {
         agent_store(&a.err[0], 2);  // (i stays past the end: the block leaves)
       }

@@ -64,3 +64,35 @@ def test_finished_instances_among_running_ones(gpu, monkeypatch, N, count, compa
     for check in (0, 3):
         states = both_routes(P, monkeypatch, cfgs, 8, bad=bad, check=check)
         assert [k for k in range(count) if states[k] == -1] == sorted(b for b in bad if b < count)
+
+
+@pytest.mark.parametrize("N,fp32", [(4096, False), (1 << 14, False), (1 << 14, True), (1 << 16, False)])
+def test_diverged_solver_goes_on_as_by_stage_launches(gpu, monkeypatch, N, fp32):
+    """A solver's slices take no notice of its power: after a round trip that is not finite the fields go through
+    the rest of the run by either route."""
+    P = gpu
+    outs = []
+    for on in ("1", "0"):
+        monkeypatch.setenv("OPO_RESIDENT", on)
+        one = []
+        for bad in (np.nan, np.inf, 1e30 if fp32 else 1e155):
+            cfg = c2(N=N, NZ=4, NRT=9)
+            p, T, w, Ap_in, Ap, As, Ai = inputs(cfg, seed=8, sigma=1e-3)
+            As = As.copy()
+            if np.isfinite(bad):  # without a pump the fields stay finite; at FP64 their power is not
+                As *= bad
+                Ap_in, Ap, Ai = 0 * Ap_in, 0 * Ap, 0 * Ai
+            else:
+                As[5] = bad
+            s = P.Solver(P.params_from(P.derive(to_args(cfg)), P.FP32C if fp32 else P.FP64))
+            s.upload(w, T, Ap_in, Ap, As, Ai)
+            s.run(0, 5)
+            one += list(s.download()) + [s.power_history(5)]
+            s.set_fields(Ap, np.zeros(N), Ai)  # a run from sound fields is sound again
+            s.run(0, 2)
+            one += list(s.download())
+            assert all(np.isfinite(f).all() for f in one[-3:])
+            s.close()
+        outs.append(one)
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b, equal_nan=True)
