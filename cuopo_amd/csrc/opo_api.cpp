@@ -14,6 +14,7 @@
 #include <cmath>
 #include <complex>
 #include <cstdint>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -2072,11 +2073,19 @@ int autotune_joint(Engine &E, int iters) {
 // With several grid sizes, autotune_joint then weighs the picks side by side.
 // The timed slices mutate the fields, so each group's state is saved before
 // and restored after, as are the settings if the tuning fails.
+// OPO_TUNE_LOG=1 writes a line per timed setting to stderr.
 int engine_autotune(Engine &E, int iters) {
-  for (size_t gi = 0; gi < E.groups.size(); ++gi) {
-    Group &g = E.groups[gi];
+  for (auto &g : E.groups)
     for (auto &I : g.inst)
       if (!I.uploaded) return fail(OPO_ERR_STATE, "autotune before upload");
+  // every instance launched (none are before the first run, and only the last
+  // ones after a compacted one): the rule that chooses the route counts them
+  E.inst_dirty = true;
+  RCHK(sync_insts(E));
+  const char *tl = std::getenv("OPO_TUNE_LOG");
+  const bool log = tl && tl[0] != '0';
+  for (size_t gi = 0; gi < E.groups.size(); ++gi) {
+    Group &g = E.groups[gi];
     // the groups of one grid size (a large one-size batch split in two) share
     // the settings tuned on the first of them
     bool shared = false;
@@ -2125,6 +2134,10 @@ int engine_autotune(Engine &E, int iters) {
       RCHK(engine_time_slices(E, g, n, &u0));
       RCHK(engine_time_slices(E, g, n, &u1));
       *us = std::min(u0, u1);
+      if (log)
+        std::fprintf(stderr, "opo autotune: N %d of %d by %s, column tile %d x %d, rows %d x %d, xcd_pack %d, phase %d: %.2f us\n",
+                     g.N, (int)g.members.size(), time_resident(E) ? "one launch" : "stages", g.ct, g.ce, g.rt, g.re,
+                     t.xcd_pack, t.phase_mode, *us);
       return OPO_OK;
     };
     opo_tuning best = base;

@@ -1,0 +1,40 @@
+"""What the autotuner times: the route that the batch's runs take, with that route's own settings."""
+import re
+
+import pytest
+
+from tests.helpers import c1, c2, inputs, to_args
+
+pytestmark = pytest.mark.gpu
+
+LINE = re.compile(r"opo autotune: N (\d+) of (\d+) by (one launch|stages), column tile (\d+) x (\d), rows (\d+) x (\d)")
+
+
+def tuned(P, monkeypatch, capfd, cfg, count, run_first=False):
+    """(by one launch, by stages): the settings timed, each (column tile, samples, row tile, samples)."""
+    monkeypatch.setenv("OPO_TUNE_LOG", "1")
+    p, T, w, Ap_in, Ap, As, Ai = inputs(cfg, seed=4, sigma=1e-3)
+    prm = P.params_from(P.derive(to_args(cfg)), P.FP64)
+    b = P.Batch([prm] * count)
+    for k in range(count):
+        b.upload(k, w, T, Ap_in, Ap, As, Ai)
+    if run_first:
+        b.run(1, check_every=0, tol=0.0)
+    capfd.readouterr()
+    b.autotune(iters=2)
+    err = capfd.readouterr().err
+    b.close()
+    out = {"one launch": set(), "stages": set()}
+    for m in LINE.finditer(err):
+        out[m.group(3)].add(tuple(int(m.group(k)) for k in (4, 5, 6, 7)))
+    return out["one launch"], out["stages"]
+
+
+@pytest.mark.parametrize("run_first", [False, True])
+@pytest.mark.parametrize("config", [c1, c2])
+def test_batch_beyond_the_one_launch_pass_tunes_all_its_tiles(gpu, monkeypatch, capfd, config, run_first):
+    """2^20 samples at 2^10 run by stages, also before the batch has run for the first time."""
+    one, stages = tuned(gpu, monkeypatch, capfd, config(N=1024, NZ=6, NRT=5), 1024, run_first)
+    assert not one
+    # 32 rows of 32 points: 64 threads of 8 samples take 16 rows, more threads all 32
+    assert {t[0] for t in stages} >= {4, 8, 16} and {t[2] for t in stages if t[3] == 8} >= {16, 32}
