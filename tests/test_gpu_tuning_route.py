@@ -38,3 +38,11 @@ def test_batch_beyond_the_one_launch_pass_tunes_all_its_tiles(gpu, monkeypatch, 
     assert not one
     # 32 rows of 32 points: 64 threads of 8 samples take 16 rows, more threads all 32
     assert {t[0] for t in stages} >= {4, 8, 16} and {t[2] for t in stages if t[3] == 8} >= {16, 32}
+
+
+@pytest.mark.parametrize("N,count", [(1 << 14, 64), (1 << 15, 1), (1 << 15, 32), (4096, 3)])
+def test_batch_within_the_pass_times_nothing_else(gpu, monkeypatch, capfd, N, count):
+    """Settings that would send the batch back to stage launches (two turns of 2^14 with 4 samples per thread are
+    four; rows of 512 points do not fit a wavefront at 4) are not tried beside the pass."""
+    one, stages = tuned(gpu, monkeypatch, capfd, c2(N=N, NZ=6, NRT=5), count)
+    assert one and not stages
