@@ -673,6 +673,12 @@ ResShape res_shape(const Engine &E, const Group &g) { return res_shape(g, res_co
 // whether full or not, and the two-launch path streams about 31 ps per sample
 // beside 7 us; the shorter estimate decides (256
 // instances of 2^14: 124 against 141 us; 71: 49 against 41).
+// Two equations stream two fields, and their nonlinear step fills the pass's
+// turns: 13 us a turn (11.5 up to 2^12, 13.5 at 2^15) against 20.5 ps beside 12
+// us.  Full turns of 2^11, 2^12, 2^14, 2^15, resident / stages: two 23.7 / 32.8,
+// 24.1 / 34.2, 26.1 / 34.5, 27.6 / 33.9; four 44.9 / 50.6, 45.4 / 51.9, 51.7 /
+// 53.4, 54.0 / 53.7; five of 2^13 63.2 / 66.6, of 2^15 67.6 / 63.7; eight 88.7 /
+// 93.1, 92.0 / 97.2, 102.6 / 97.1, 107.3 / 97.1.
 // FP32C streams half the bytes on the two-launch path and the pass is bound by
 // arithmetic there, so it ends at 2^19 samples (1.05 to 1.7 times; 0.5 to 1.2
 // beyond); with 4 samples per thread at 2^15 its 128 tiles per stage lose at
@@ -680,7 +686,12 @@ ResShape res_shape(const Engine &E, const Group &g) { return res_shape(g, res_co
 // Several grid sizes run side by side on their streams, where the passes would
 // run one after another (0.8 to 1.0 times).
 constexpr long long kResTurn = 1LL << 19;  // samples of one turn of every XCD's teams
-constexpr double kResTurnUs = 16.5, kStreamUs = 7.0, kStreamUsPerSample = 31e-6;
+double res_turn_us(const Group &g) {
+  return g.NF == 3 ? 16.5 : g.N <= (1 << 12) ? 11.5 : g.N < (1 << 15) ? 13.0 : 13.5;
+}
+double stream_us(const Group &g, long long samples) {
+  return g.NF == 3 ? 7.0 + 31e-6 * (double)samples : 12.0 + 20.5e-6 * (double)samples;
+}
 
 // One instance of 2^15 samples or more with 8 samples per thread in the rows:
 // the whole chip works on it (opo_chip.h: 1.15 to 1.45 times the two-launch
@@ -705,7 +716,7 @@ bool engine_resident(const Engine &E) {
   if (samples <= kResTurn) return true;
   const ResShape r = res_shape(g, count);
   const int turn = r.teams * opo::kXcds;
-  return (count + turn - 1) / turn * kResTurnUs < kStreamUs + kStreamUsPerSample * (double)samples;
+  return (count + turn - 1) / turn * res_turn_us(g) < stream_us(g, samples);
 }
 
 // 8-byte words of the counters that a pass with this many team lines uses

@@ -46,3 +46,13 @@ def test_batch_within_the_pass_times_nothing_else(gpu, monkeypatch, capfd, N, co
     four; rows of 512 points do not fit a wavefront at 4) are not tried beside the pass."""
     one, stages = tuned(gpu, monkeypatch, capfd, c2(N=N, NZ=6, NRT=5), count)
     assert one and not stages
+
+
+@pytest.mark.parametrize("config,N,count,by_pass", [
+    (c1, 1 << 14, 128, True), (c1, 1 << 14, 256, False), (c1, 1 << 11, 2048, True),
+    (c2, 1 << 14, 256, True), (c2, 1 << 14, 40, False), (c1, 1 << 14, 40, False)])
+def test_route_follows_the_equations(gpu, monkeypatch, capfd, config, N, count, by_pass):
+    """Eight turns of 2^14 are the faster route at three equations (122 against 137 us a slice), not at two (103
+    against 97), where they still are at 2^11 (89 against 93)."""
+    one, stages = tuned(gpu, monkeypatch, capfd, config(N=N, NZ=6, NRT=5), count)
+    assert bool(one) == by_pass and bool(stages) != by_pass
