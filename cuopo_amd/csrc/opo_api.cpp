@@ -1660,7 +1660,12 @@ int engine_time_stages(Engine &E, Group &g, int iters, double *col_us, double *r
 // FP32C is tuned on the two-launch path and its per-field column stage even
 // where the run takes the resident pass or wavefront tiles: the samples per
 // thread and the phase source also decide how its results round (1e-4 over
-// thousands of slices), and every path then rounds alike.
+// thousands of slices), and every path then rounds alike.  What that costs
+// where the run is a one-launch pass, against its fastest setting: up to 7%
+// below a full turn; with a full turn of 2^12 to 2^15, where 8 samples per
+// thread would do in one turn what 4 take two for, up to 1.9 times (32 of 2^14
+// 19.9 against 12.1 us a slice, 8 of 2^15 15.9 against 8.6); one instance of
+// 2^16 1.2 times.
 bool time_resident(const Engine &E) { return engine_resident(E) && !E.fp32; }
 
 // n slices as a round trip of the group runs them, for timing: back-to-back

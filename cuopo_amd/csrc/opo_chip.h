@@ -19,7 +19,16 @@
 // Memory order.  Blocks read what other XCDs wrote, so the fields are stored at
 // agent scope as well as loaded (sc1: past the XCD's L2); a block waits for its
 // stores (vmcnt), then adds one to one of 64 counters, which a wavefront of
-// every waiting block polls, a counter a lane.  Load, store and barrier of 3 MB
+// every waiting block polls, a counter a lane.  What that rests on, in the
+// AMDGPU backend's memory model for gfx942 and gfx950: stores and loads marked
+// sc1 are the model's relaxed atomic accesses of agent scope, coherent at every
+// address over all L2s of the device; and vmcnt reaches zero when a store is
+// complete at its scope, so the counter moves after the data.  The model's
+// agent fences add a write-back and an invalidation of the L2, for accesses
+// without sc1, which the fields do not have here.  It names accesses of up to 8
+// bytes; a 16-byte one carries the same bits and is taken as two of those: no
+// more is needed, as the counter orders them.  The tests compare every grid,
+// type and equation set with the stage launches bit for bit.  Load, store and barrier of 3 MB
 // of fields (2^16, FP64) take 2.9 us on 192 blocks so; with one counter per XCD
 // and one for the XCDs 3.3, with a flag per block 3.2 to 4.1, with one counter
 // 6.8 (256 blocks).

@@ -112,10 +112,9 @@ constexpr int kXcds = 8, kMaxTeams = 32;  // teams per XCD
 struct alignas(128) ResLine {
   unsigned v;
 };
-struct alignas(128) ResLine128 { unsigned v; };
 constexpr int kTeamCounters = 8;
 struct ResTeam {
-  ResLine128 part[kTeamCounters];        // stages finished, summed over the team's blocks (block b: part b mod kTeamCounters)
+  ResLine part[kTeamCounters];        // stages finished, summed over the team's blocks (block b: part b mod kTeamCounters)
   alignas(128) unsigned long long cur;   // (turn << 32) | instance the team works on
 };
 struct ResSync {
@@ -138,10 +137,9 @@ struct ResArgs {
   void *sync;        // ResSync
   int *err;          // set on a time-out, never cleared by a kernel
 };
-// threads per block of the resident pass
-constexpr int res_max_threads(int, int) { return 768; }
-bool resident_supported(int N1, int N2, int ce, int re);
+constexpr int kResThreads = 768;  // per block of the resident pass, at most
 constexpr unsigned kMaxPolls = 1u << 23;  // seconds: a poll takes a few hundred ns
+bool resident_supported(int N1, int N2, int ce, int re);
 constexpr int kChipBlocks = 256;  // one per CU
 constexpr int kChipCounters = 64;
 bool chip_supported(int N1, int N2, int ce, int re, int fp32);

@@ -737,7 +737,7 @@ int launch_resident(int fp32, int N1, int N2, int NF, int ce, int re, const OpoI
   return f(N1, N2, ce, re, insts, a, grid, (hipStream_t)stream);
 }
 
-// One instance of N = 2^16 .. 2^18 over all CUs (opo_chip_*.hip), 8 samples per thread in the rows.
+// One instance of N = 2^15 .. 2^18 over all CUs (opo_chip_*.hip), 8 samples per thread in the rows.
 int launch_chip_f64(int, int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
 int launch_chip_f32(int, int, int, int, const OpoInst *, const ResArgs &, hipStream_t);
 

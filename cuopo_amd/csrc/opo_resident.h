@@ -276,7 +276,7 @@ __device__ __forceinline__ bool col_tile(const FieldBuf<V> &in, const ResArgs &a
 }
 
 template <typename T, int N1, int N2, int NF, int EC, int ER>
-__global__ __launch_bounds__(res_max_threads(EC, ER)) void resident_pass(const OpoInst *__restrict__ insts, ResArgs a) {
+__global__ __launch_bounds__(kResThreads) void resident_pass(const OpoInst *__restrict__ insts, ResArgs a) {
   using V = typename vec2<T>::type;
   constexpr int T1 = N1 / EC, T2 = N2 / ER;
   constexpr int CT = 64 / T1, RT = 64 / T2;
@@ -444,7 +444,7 @@ int launch_resident_k(const OpoInst *insts, const ResArgs &a, int grid, hipStrea
   using V = typename vec2<T>::type;
   const int threads = 64 * NF * a.sub;
   const size_t lds = ((size_t)N1 + (size_t)a.sub * res_tile_elems<NF, EC, ER>()) * sizeof(V);
-  if (a.sub < 1 || threads > res_max_threads(EC, ER) || lds > kMaxDynLds || grid < kXcds || a.teams < 1 ||
+  if (a.sub < 1 || threads > kResThreads || lds > kMaxDynLds || grid < kXcds || a.teams < 1 ||
       a.teams > kMaxTeams)
     return (int)hipErrorInvalidValue;
   auto kern = &resident_pass<T, N1, N2, NF, EC, ER>;
