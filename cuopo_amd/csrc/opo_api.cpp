@@ -115,6 +115,7 @@ struct Group {
   bool any_gdd = false;
   opo::ResSync *d_sync = nullptr;  // counters of the resident pass; null: no resident pass for this group
   int *d_err = nullptr;            // its time-out flag
+  bool passes = false;             // a pass has been launched or captured, so the flag may be set
   std::vector<void *> allocs;
   // no-allocation mode: device memory comes from the caller's buffers (fields,
   // pump) and a bump pool over the static scratch array instead of hipMalloc
@@ -746,6 +747,7 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
   a.spread = total < r.teams * opo::kXcds;
   // consecutive handles prefer different XCDs
   a.prefer = (int)((reinterpret_cast<uintptr_t>(g.d_insts) >> 12) % opo::kXcds);
+  g.passes = true;
   a.polls = E.polls;
   a.always = E.solver;
   a.sync = g.d_sync;
@@ -766,7 +768,7 @@ int emit_resident(Engine &E, Group &g, int nz, bool alone = false) {
 int check_resident(Engine &E) {
   bool timed_out = false;
   for (auto &g : E.groups) {
-    if (!g.d_err) continue;
+    if (!g.passes) continue;
     int err = 0;
     HIPCHK(hipMemcpyAsync(&err, g.d_err, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     HIPCHK(hipStreamSynchronize(E.stream));
